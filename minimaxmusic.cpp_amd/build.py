@@ -46,8 +46,8 @@ HOST_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall", f"-I{GGML_INC}", f"-I{ROOT 
 # (library, compiler, sources, link flags)
 LIBS = [
     ("libmmhip.so", "hip",
-     ["csrc/k_quant.hip", "csrc/k_gemv.hip", "csrc/k_gemm.hip", "csrc/k_fa_decode.hip", "csrc/k_fa_mfma.hip",
-      "csrc/k_glue.hip", "csrc/k_synth.hip", "csrc/mmhip_api.hip"], []),
+     ["csrc/k_quant.hip", "csrc/k_gemv.hip", "csrc/k_gemm.hip", "csrc/k_gemm_skinny.hip", "csrc/k_gemm_pipe.hip",
+      "csrc/k_fa_decode.hip", "csrc/k_fa_mfma.hip", "csrc/k_glue.hip", "csrc/k_synth.hip", "csrc/mmhip_api.hip"], []),
     # stand-in for libggml-base (ggml is not vendored by the reference)
     ("libggml-base.so", "host", ["ggml/src/ggml_core.cpp", "ggml/src/gguf.cpp"], ["-ldl"]),
     # the MI355X ggml backend, on top of the two above

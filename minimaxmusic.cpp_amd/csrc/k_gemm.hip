@@ -18,32 +18,18 @@
 #include <type_traits>
 #include <unordered_map>
 
-#include "mmhip_device.h"
-#include "mmhip_internal.h"
+#include "k_gemm_common.h"
 
 namespace mmhip {
 
 constexpr int GM_BK = 64;
-constexpr int GM_LS = GM_BK + 8;  // LDS row stride in halves (144 bytes)
-
-__device__ __forceinline__ float16_t gm_mfma(half8_t a, half8_t b, float16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-// The same product on bf16 operands (carried as 16-bit patterns in half8_t):
-// bf16 x bf16 products are exact in f32 and accumulate in f32.
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-
-__device__ __forceinline__ float16_t gm_mfma_bf16(half8_t a, half8_t b, float16_t c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
-                                                   0, 0, 0);
-}
 
 // Raw bytes a thread needs for its half row (32 weights) of one K step.
 struct WRaw {
     int4_t   q0, q1;     // quant bytes (Q5_K: q1 = the fifth-bit bytes)
     uint32_t s0, s1, s2;  // Q4_K / Q5_K scales; Q6_K high bits (with dm)
     uint32_t dm;          // f16 scale(s)
+    uint32_t sc, d;       // Q6_K: the scales of the step's two quarters, f16 d
 };
 
 // Thread t of the workgroup owns weight row (t / 2) of the tile and the half
@@ -84,41 +70,62 @@ __device__ __forceinline__ void w_load(WRaw & w, const uint8_t * row, int64_t K,
         w.s1 = (uint32_t) qh.y;
         w.s2 = (uint32_t) qh.z;
         w.dm = (uint32_t) qh.w;
+        w.sc = *(const uint32_t *) (row + K / 2 + K / 4 + sb * 16 + hf * 8 + 2 * tq);
+        w.d  = *(const uint16_t *) (row + K / 2 + K / 4 + K / 16 + 2 * sb);
     }
 }
 
-// Byte e of a 16-byte load, as the format's signed / unsigned value.  The
-// bytes are taken from the 32-bit words with shifts at the point of use: a
-// byte-pointer view of the loaded vector makes the compiler unpack it right
-// after the load, which forces the wait for that load before the MFMA work
-// that should hide it.
-__device__ __forceinline__ int byte_s(const int4_t & v, int e) {
-    return (int) (int8_t) (v[e >> 2] >> (8 * (e & 3)));
-}
+// The bytes of the loaded quants are taken from the 32-bit words at the point
+// of use: a byte-pointer view of the loaded vector makes the compiler unpack
+// it right after the load, which forces the wait for that load before the
+// MFMA work that should hide it.
 
-__device__ __forceinline__ int byte_u(const int4_t & v, int e) {
-    return (v[e >> 2] >> (8 * (e & 3))) & 0xff;
-}
+// f((float) byte) for the four bytes of x, in f32, rounded to f16 by the packed
+// conversion
+typedef float float2_t __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ int byte_u32(const uint32_t (&w)[4], int e) {
-    return (int) ((w[e >> 2] >> (8 * (e & 3))) & 0xff);
+template <class F> __device__ __forceinline__ void dq_bytes(uint32_t x, half8_t & o, int at, F f) {
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const float2_t v = { f((float) ((x >> (8 * i)) & 0xff)), f((float) ((x >> (8 * i + 8)) & 0xff)) };
+        const half2_t  h = __builtin_convertvector(v, half2_t);
+        o[at + i]        = h[0];
+        o[at + i + 1]    = h[1];
+    }
 }
 
 // Dequantise the thread's 32 weights (f32 exact, then f16) into four 16-byte
 // chunks o[0..3] and name the chunk index (0..7) of the 64-wide K step each
 // one belongs to (Q8_0: 4*half + c; Q4_K / Q6_K: low nibbles or first
 // quarter at 2*half + {0,1}, high nibbles or second quarter at 4 + 2*half +
-// {0,1}).
+// {0,1}).  The values are the GGUF definitions' f32 results rounded once to
+// f16, reached in two or three VALU operations each (ten in the form that
+// widened every quant to f32 and scaled it there), whose count set the pace
+// of the register-staged kernel:
+//   Q8_0      d * q as a packed f16 product: q is exact in f16, so the product
+//             is the exact one rounded once, as the f32 product's rounding is
+//   Q4_K/Q5_K d1 * q - m1 as one fma: d1 = d * sc and d1 * q are exact in f32
+//             (at most 22 bits), so the fma rounds where the difference does
+//   Q6_K      ds * (q - 32) as fma(q, ds, -32 ds): 32 ds is exact, so the fma
+//             rounds the exact product once, as the product does
 template <int WT>
-__device__ __forceinline__ void w_dequant(const WRaw & w, const uint8_t * row, int64_t K, int k0, int half,
-                                          half8_t (&o)[4], int (&chunk)[4]) {
+__device__ __forceinline__ void w_dequant(const WRaw & w, int k0, int half, half8_t (&o)[4], int (&chunk)[4]) {
 #pragma clang fp contract(off)
     if constexpr (WT == TYPE_Q8_0) {
-        const float d = h2f((uint16_t) w.dm);
+        const _Float16 d   = __builtin_bit_cast(_Float16, (uint16_t) w.dm);
+        const half2_t  dd  = { d, d };
+        const half2_t  off = { (_Float16) 1152.0f, (_Float16) 1152.0f };
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            o[i / 8][i % 8]     = (_Float16) (d * (float) byte_s(w.q0, i));
-            o[2 + i / 8][i % 8] = (_Float16) (d * (float) byte_s(w.q1, i));
+        for (int i = 0; i < 8; i++) {
+            const uint32_t u = (uint32_t) (i < 4 ? w.q0[i & 3] : w.q1[i & 3]) ^ 0x80808080u;  // q + 128
+            // 0x6400 | byte is the f16 1024 + byte
+            const half2_t a = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u));
+            const half2_t b = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u));
+            const half2_t x = (a - off) * dd, y = (b - off) * dd;
+            o[i / 2][4 * (i & 1)]     = x[0];
+            o[i / 2][4 * (i & 1) + 1] = x[1];
+            o[i / 2][4 * (i & 1) + 2] = y[0];
+            o[i / 2][4 * (i & 1) + 3] = y[1];
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -134,51 +141,42 @@ __device__ __forceinline__ void w_dequant(const WRaw & w, const uint8_t * row, i
         const float d1 = d * (float) sc_lo, m1 = dmin * (float) mn_lo;
         const float d2 = d * (float) sc_hi, m2 = dmin * (float) mn_hi;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int q  = byte_u(w.q0, i);
-            int       ql = q & 15, qh = q >> 4;
+        for (int i = 0; i < 4; i++) {
+            uint32_t ql = (uint32_t) w.q0[i] & 0x0f0f0f0fu, qh = ((uint32_t) w.q0[i] >> 4) & 0x0f0f0f0fu;
             if constexpr (WT == TYPE_Q5_K) {
-                const int h = byte_u(w.q1, i);
-                ql |= ((h >> (2 * c)) & 1) << 4;
-                qh |= ((h >> (2 * c + 1)) & 1) << 4;
+                const uint32_t h = (uint32_t) w.q1[i] >> (2 * c);
+                ql |= (h & 0x01010101u) << 4;
+                qh |= ((h >> 1) & 0x01010101u) << 4;
             }
-            o[i / 8][i % 8]     = (_Float16) (d1 * (float) ql - m1);
-            o[2 + i / 8][i % 8] = (_Float16) (d2 * (float) qh - m2);
+            dq_bytes(ql, o[i / 2], 4 * (i & 1), [&](float q) { return __builtin_fmaf(q, d1, -m1); });
+            dq_bytes(qh, o[2 + i / 2], 4 * (i & 1), [&](float q) { return __builtin_fmaf(q, d2, -m2); });
         }
         chunk[0] = 2 * half;
         chunk[1] = 2 * half + 1;
         chunk[2] = 4 + 2 * half;
         chunk[3] = 4 + 2 * half + 1;
     } else {
-        const int       sb = k0 >> 8, hf = (k0 & 255) >> 7, tq = (k0 & 127) >> 5;
-        const float     d  = h2f(*(const uint16_t *) (row + K / 2 + K / 4 + K / 16 + 2 * sb));
-        const int8_t *  sc = (const int8_t *) (row + K / 2 + K / 4) + sb * 16 + hf * 8;
+        const int       tq = (k0 & 127) >> 5;
+        const float     d  = h2f((uint16_t) w.d);
         const uint32_t  qhw[4] = { w.s0, w.s1, w.s2, w.dm };
         // element l0 + i of quarter t has scale index 2t + (l0 + i) / 16 = 2t + half
-        const float ds0 = d * (float) sc[2 * tq + half];
-        const float ds1 = d * (float) sc[2 * (tq + 1) + half];
+        const float ds0 = d * (float) (int8_t) (w.sc >> (8 * half));
+        const float ds1 = d * (float) (int8_t) (w.sc >> (16 + 8 * half));
+        const float of0 = -32.0f * ds0, of1 = -32.0f * ds1;
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int qa = byte_u(w.q0, i), qb = byte_u(w.q1, i), qh = byte_u32(qhw, i);
-            const int lo0 = tq == 0 ? (qa & 15) : (qa >> 4);
-            const int lo1 = tq == 0 ? (qb & 15) : (qb >> 4);
-            const int h0  = (qh >> (2 * tq)) & 3;
-            const int h1  = (qh >> (2 * tq + 2)) & 3;
-            o[i / 8][i % 8]     = (_Float16) (ds0 * (float) ((lo0 | (h0 << 4)) - 32));
-            o[2 + i / 8][i % 8] = (_Float16) (ds1 * (float) ((lo1 | (h1 << 4)) - 32));
+        for (int i = 0; i < 4; i++) {
+            // tq = 0: low nibbles and high bits 0..3; tq = 2: high nibbles, bits 4..7
+            const uint32_t h  = qhw[i] >> (2 * tq);
+            const uint32_t q0 = (((uint32_t) w.q0[i] >> (2 * tq)) & 0x0f0f0f0fu) | ((h & 0x03030303u) << 4);
+            const uint32_t q1 = (((uint32_t) w.q1[i] >> (2 * tq)) & 0x0f0f0f0fu) | (((h >> 2) & 0x03030303u) << 4);
+            dq_bytes(q0, o[i / 2], 4 * (i & 1), [&](float q) { return __builtin_fmaf(q, ds0, of0); });
+            dq_bytes(q1, o[2 + i / 2], 4 * (i & 1), [&](float q) { return __builtin_fmaf(q, ds1, of1); });
         }
         chunk[0] = 2 * half;
         chunk[1] = 2 * half + 1;
         chunk[2] = 4 + 2 * half;
         chunk[3] = 4 + 2 * half + 1;
     }
-}
-
-// Consecutive work items go to one XCD (workgroups are dealt round-robin over
-// the 8 XCDs), so the workgroups sharing an activation tile share an L2.
-__device__ __forceinline__ int64_t gm_xcd_remap(int64_t lin, int64_t total) {
-    const int64_t per = total / 8;
-    return lin >= per * 8 ? lin : (lin % 8) * per + lin / 8;
 }
 
 // The activation tile reaches LDS without passing through registers:
@@ -191,14 +189,6 @@ typedef __attribute__((address_space(3))) _Float16 lds_half_t;
 
 __device__ __forceinline__ void dma16(const void * src, uint32_t lds_addr) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory", "m0");
-}
-
-// Tiles in LDS are unpadded rows of 64 halves (8 chunks of 16 bytes) with
-// chunk c of row r stored at chunk c ^ (r & 7): the 32 rows an MFMA operand
-// read touches then spread over all banks.
-template <int BK>
-__device__ __forceinline__ int swz(int r, int c) {
-    return r * BK + 8 * (c ^ (r & 7));
 }
 
 // Rows of 32 halves (the f16-weight ring's K step): chunk c of row r at
@@ -268,34 +258,9 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_q(const uint8_t * __restrict__
     _Float16 * sX = g_lds;            // 2 stages
     _Float16 * sW = g_lds + 2 * TIX;  // 2 buffers
 
-    // consecutive work items (one XCD, one L2) share the operand that is
-    // re-read most: the weight tile when there are more weight tiles than
-    // token tiles (m_fast: its token tiles run together), else the
-    // activation tiles, in groups of GM_GROUP token tiles with the token tile
-    // fastest, so that the workgroups running together on an XCD cover a
-    // block of GM_GROUP token tiles by several weight tiles and each weight
-    // tile is fetched once per group rather than once per token tile
-    // split-K: work items (part, tile), the parts of one tile n_base apart
-    constexpr int GM_GROUP = 4;
-    const int64_t n_base  = n_tiles / spl.n;
-    const int64_t lin     = gm_xcd_remap(blockIdx.x, n_tiles);
-    const int     kpart   = (int) (lin / n_base);
-    const int64_t work    = lin % n_base;
-    const int64_t n_mt    = n_base / n_ntiles;
-    const bool    m_fast  = n_ntiles > n_mt;
-    int64_t       tm, tn;  // token tile, weight tile
-    if (m_fast) {
-        tm = work % n_mt;
-        tn = work / n_mt;
-    } else {
-        const int64_t gsz = (int64_t) GM_GROUP * n_ntiles;
-        const int64_t g   = work / gsz, r = work % gsz;
-        const int64_t gw  = min((int64_t) GM_GROUP, n_mt - g * GM_GROUP);
-        tm                = g * GM_GROUP + r % gw;
-        tn                = r / gw;
-    }
-    const int64_t m0 = tm * BM;
-    int64_t       n0 = tn * BT;
+    int64_t m0, n0;
+    int     kpart;
+    gm_tile(n_ntiles, n_tiles, spl.n, BM, BT, m0, n0, kpart);
     if (mul.n > 0) {
         // several weight matrices: this tile's rows come from matrix n0 / Nper
         const int mi = (int) (n0 / mul.Nper);
@@ -361,7 +326,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_q(const uint8_t * __restrict__
         for (int u = 0; u < SUB; u++) {
             half8_t o[4];
             int     ch[4];
-            w_dequant<WT>(wr[u], wrow, K, k0 + GM_BK * u, shalf, o, ch);
+            w_dequant<WT>(wr[u], k0 + GM_BK * u, shalf, o, ch);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 *(half8_t *) &sW[buf * TIL + swz<BK>(srow, ch[j] + 8 * u)] = w_ok ? o[j] : half8_t{};
@@ -609,165 +574,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_q(const uint8_t * __restrict__
     }
     }
 
-    // C[i = token][j = weight row]: lane holds row j = lq, tokens 8(r/4) + 4hh + r%4.
-    // Each epilogue runs branch-free on whole tiles (all but the last row and
-    // column of tiles): at the joins of per-element bounds branches the
-    // compiler waits for every store in flight, one wait per element.
-    const int64_t mw     = m0 + wm * (BM / WM) + 4 * hh;  // token of register 0 in block i = 0
-    const bool    full_m = m0 + BM <= M;
-    if constexpr (GLU) {
-        // pair p of this wave: value block 2p, gate block 2p + 1, SwiGLU column j
-        constexpr int NP = NB / 2;
-        int64_t       jp[NP];
-        float         bv[NP], bg[NP];
-#pragma unroll
-        for (int q = 0; q < NP; q++) {
-            jp[q]            = n0 / 2 + wn * (BT / WN / 2) + q * 32 + lq;
-            const bool    ok = jp[q] < glu.F;
-            const int64_t rv = glu.swapped ? glu.F + jp[q] : jp[q];  // value row
-            const int64_t rg = glu.swapped ? jp[q] : glu.F + jp[q];  // gate row
-            bv[q]            = bias && ok ? bias[rv] : 0.0f;
-            bg[q]            = bias && ok ? bias[rg] : 0.0f;
-        }
-        // the bias in registers before any store: a use behind a store's
-        // bounds branch would otherwise wait for all stores in flight
-        __builtin_amdgcn_s_waitcnt(0);
-        auto go = [&](auto full_c) {
-            constexpr bool FULL = decltype(full_c)::value;
-#pragma unroll
-            for (int q = 0; q < NP; q++) {
-                const int64_t j = jp[q];
-                if (j >= glu.F) {
-                    continue;
-                }
-#pragma unroll
-                for (int i = 0; i < MB; i++) {
-                    float o[16];
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        float v = acc[i][2 * q][r], g = acc[i][2 * q + 1][r];
-                        if (bias) {
-                            v = v + bv[q];
-                            g = g + bg[q];
-                        }
-                        const float silu = g / (1.0f + expf(-g));
-                        o[r]             = silu * v;
-                    }
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int64_t m = mw + i * 32 + 8 * (r / 4) + (r % 4);
-                        if (FULL || m < M) {
-                            if (glu.h) {
-                                glu.h[m * glu.F + j] = o[r];
-                            }
-                            if (glu.hh) {
-                                glu.hh[m * glu.F + j] = (_Float16) o[r];
-                            }
-                        }
-                    }
-                }
-            }
-        };
-        if (full_m) {
-            go(std::integral_constant<bool, true>{});
-        } else {
-            go(std::integral_constant<bool, false>{});
-        }
-        return;
-    }
-    const int64_t nl   = n0 + wn * (BT / WN) + lq;  // this lane's column in weight block 0
-    const bool    full = full_m && n0 + BT <= N;
-    if (spl.n > 1) {
-        // partial sums of this K part; the reduce kernel adds the ADDs
-        float * pp = spl.part + (int64_t) kpart * M * N;
-        auto    go = [&](auto full_c) {
-            constexpr bool FULL = decltype(full_c)::value;
-#pragma unroll
-            for (int i = 0; i < MB; i++) {
-#pragma unroll
-                for (int j = 0; j < NB; j++) {
-                    const int64_t n = nl + 32 * j;
-                    if (!FULL && n >= N) {
-                        continue;
-                    }
-#pragma unroll
-                    for (int r = 0; r < 16; r++) {
-                        const int64_t m = mw + i * 32 + 8 * (r / 4) + (r % 4);
-                        if (FULL || m < M) {
-                            pp[m * N + n] = acc[i][j][r];
-                        }
-                    }
-                }
-            }
-        };
-        if (full) {
-            go(std::integral_constant<bool, true>{});
-        } else {
-            go(std::integral_constant<bool, false>{});
-        }
-        return;
-    }
-    // Epilogue: the bias ADD, then the residual ADD, each rounded as its op.
-    // The bias is loaded once per column, and each 32 x 32 block's residual
-    // values are loaded before the previous block's stores are issued (loads
-    // and stores share one completion counter, so a load issued behind
-    // stores would wait for them too).  In place (res == y) every element is
-    // read before this thread writes it, and no other thread touches it.
-    float bn[NB];
-#pragma unroll
-    for (int j = 0; j < NB; j++) {
-        bn[j] = bias && nl + 32 * j < N ? bias[nl + 32 * j] : 0.0f;
-    }
-    __builtin_amdgcn_s_waitcnt(0);  // the bias in registers before any store
-    auto go = [&](auto full_c) {
-        constexpr bool FULL = decltype(full_c)::value;
-        float          rv[16];
-        auto           rload = [&](int b) {
-            const int64_t n = nl + 32 * (b % NB);
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int64_t m = mw + (b / NB) * 32 + 8 * (r / 4) + (r % 4);
-                rv[r]           = FULL || (m < M && n < N) ? res[m * ldr + n] : 0.0f;
-            }
-        };
-        if (res) {
-            rload(0);
-        }
-#pragma unroll
-        for (int b = 0; b < MB * NB; b++) {
-            const int     i = b / NB, j = b % NB;
-            const int64_t n = nl + 32 * j;
-            float         v[16];
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                v[r] = bias ? acc[i][j][r] + bn[j] : acc[i][j][r];
-            }
-            if (res) {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    v[r] = rv[r] + v[r];
-                }
-                if (b + 1 < MB * NB) {
-                    rload(b + 1);
-                }
-            }
-            if (!FULL && n >= N) {
-                continue;
-            }
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int64_t m = mw + i * 32 + 8 * (r / 4) + (r % 4);
-                if (FULL || m < M) {
-                    y[m * ldy + n] = v[r];
-                }
-            }
-        }
-    };
-    if (full) {
-        go(std::integral_constant<bool, true>{});
-    } else {
-        go(std::integral_constant<bool, false>{});
-    }
+    gm_epilogue<MB, NB, BM, BT, WM, WN, GLU>(acc, m0, n0, N, M, wave, lane, bias, res, ldr, y, ldy, glu, spl, kpart);
 }
 
 // Split-K reduction: y[m, n] = ((part_0 + part_1 + ...) + bias[n]) + res[m, n],
@@ -804,8 +611,11 @@ __global__ void k_splitk_reduce(const float * __restrict__ part, int nparts, int
 // [M, K] copy: 8 elements per thread per pass.
 __device__ __forceinline__ void x_to_f16_part(const float * __restrict__ x, int64_t ldx, int64_t K, int64_t n8,
                                               _Float16 * __restrict__ xh, int64_t t0, int64_t stride) {
+    const uint32_t k8 = (uint32_t) (K / 8);
     for (int64_t t = t0; t < n8; t += stride) {
-        const int64_t  e = t * 8, m = e / K, k = e % K;
+        // a 64-bit division costs more than the conversion
+        const int64_t  m = n8 < (1ll << 32) ? (uint32_t) t / k8 : t / k8;
+        const int64_t  e = t * 8, k = e - m * K;
         const float4_t a = *(const float4_t *) (x + m * ldx + k);
         const float4_t b = *(const float4_t *) (x + m * ldx + k + 4);
         half8_t        o;
@@ -827,8 +637,10 @@ __global__ void k_x_to_f16(const float * __restrict__ x, int64_t ldx, int64_t K,
 // packed [M, K] copy of 16-bit patterns, 8 elements per thread per pass.
 __global__ void k_x_to_bf16(const float * __restrict__ x, int64_t ldx, int64_t K, int64_t n8,
                             uint16_t * __restrict__ xb) {
+    const uint32_t k8 = (uint32_t) (K / 8);
     for (int64_t t = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; t < n8; t += (int64_t) gridDim.x * blockDim.x) {
-        const int64_t  e = t * 8, m = e / K, k = e % K;
+        const int64_t m = n8 < (1ll << 32) ? (uint32_t) t / k8 : t / k8;
+        const int64_t e = t * 8, k = e - m * K;
         const float4_t a = *(const float4_t *) (x + m * ldx + k);
         const float4_t b = *(const float4_t *) (x + m * ldx + k + 4);
         uint32_t       o[4];
@@ -852,15 +664,16 @@ __device__ __forceinline__ void w_to_f16_part(const uint8_t * __restrict__ W, in
         return;
     }
     const int       half = (int) (t & 1);
-    const int64_t   st   = (t >> 1) % nsteps;
-    const int64_t   row  = (t >> 1) / nsteps;
+    const int64_t   u    = t >> 1;
+    const int64_t   row  = N * nsteps < (1ll << 32) ? (uint32_t) u / (uint32_t) nsteps : u / nsteps;
+    const int64_t   st   = u - row * nsteps;
     const uint8_t * wr   = W + row * rs;
     const int       k0   = (int) (st * GM_BK);
     WRaw            w;
     w_load<WT>(w, wr, K, k0, half);
     half8_t o[4];
     int     ch[4];
-    w_dequant<WT>(w, wr, K, k0, half, o, ch);
+    w_dequant<WT>(w, k0, half, o, ch);
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         *(half8_t *) (wh + row * K + k0 + 8 * ch[j]) = o[j];
@@ -955,12 +768,18 @@ static int launch_gemm(int wtype, const uint8_t * W, int64_t N, int64_t K, int64
                          : go(k_gemm_q<TYPE_F16, NW, WM, BK, BM, false, true, WIDE>);
     } else {
         if (glu.F > 0) {
+            if constexpr (NW == 4) {
+                return go(k_gemm_q<TYPE_Q8_0, NW, WM, BK, BM, true>);
+            }
             switch (wtype) {
                 case TYPE_Q8_0: return go(k_gemm_q<TYPE_Q8_0, NW, WM, BK, BM, true>);
                 case TYPE_Q4_K: return go(k_gemm_q<TYPE_Q4_K, NW, WM, BK, BM, true>);
                 case TYPE_Q5_K: return go(k_gemm_q<TYPE_Q5_K, NW, WM, BK, BM, true>);
                 default: return go(k_gemm_q<TYPE_Q6_K, NW, WM, BK, BM, true>);
             }
+        }
+        if constexpr (NW == 4) {
+            return go(k_gemm_q<TYPE_Q8_0, NW, WM, BK, BM, false>);
         }
         switch (wtype) {
             case TYPE_Q8_0: return go(k_gemm_q<TYPE_Q8_0, NW, WM, BK, BM, false>);
@@ -971,68 +790,58 @@ static int launch_gemm(int wtype, const uint8_t * W, int64_t N, int64_t K, int64
     }
 }
 
-// Tile configuration by shape (activations already f16, rows of K).
+// The split-K sums added in order, with the ADDs.
+static int splitk_reduce(const GemmSplit & spl, int64_t M, int64_t N, const float * bias, const float * res,
+                         int64_t ldr, float * y, int64_t ldy, hipStream_t stream) {
+    const int64_t nt = M * (N / 4);
+    const int64_t nb = (nt + 255) / 256;
+    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned) (nb < 16384 ? nb : 16384)), dim3(256), 0, stream,
+                       (const float *) spl.part, spl.n, M, N, bias, res, ldr, y, ldy);
+    return check_launch("mul_mat gemm: split-K reduce");
+}
+
+// Kernel and tile by shape (activations already 16 bits, rows of K).  wtype
+// F16 / BF16: 16-bit weight rows rs bytes apart.  Every choice adds the
+// products in the same order, so the results do not depend on it.  The times
+// compared (us) are gemm_p_us's and, on the rounds of 256 tiles they take,
+//   256 x 256 DMA ring (16-bit rows)      2.1 per 64-column step and round
+//   256 x 256 register-staged (quantised) 2.3
+//   64 x 128 DMA ring (16-bit rows)       0.3 + 0.0018 per tile a step
+// (16384 x 2048 f16 rows at 690 tokens: 60 us on 192-token tiles, 95 on the
+// 64 x 128 ring; 2048 x 2048 at 333: 18 on the small ring, 23 on 64 tokens;
+// 24576 x 4096 Q8_0 at 2000: 447 register-staged, 480 on 192 tokens, at 690
+// 184 on 192 tokens, 258 register-staged).
 static int gemm_launch(int wtype, const uint8_t * wb, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
                        const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
-                       const GemmMulti & mul, const GemmSplit & spl, hipStream_t stream, bool wh = false) {
-    const int64_t tiles256 = ((N + 255) / 256) * ((M + 255) / 256);
-    if (wh) {
-        // f16 weight rows (row stride K): the DMA ring on the same tile choice.
-        // 192-token tiles (3/4 of the work of a 256-token tile) where they
-        // take fewer rounds of the 256 CUs by that weight: the DiT's 1380
-        // tokens fill 8 of them (5.4 of 256) and its projections' grids of
-        // 144 to 384 tiles of 256 run a partly filled round
-        const int64_t nn     = (N + 255) / 256;
-        const int64_t r256   = (nn * ((M + 255) / 256) * spl.n + 255) / 256;
-        const int64_t r192   = (nn * ((M + 191) / 192) * spl.n + 255) / 256;
-        const bool    bm192  = 3 * r192 < 4 * r256;
-        auto          wide   = [&](const float * bi, const float * re, int64_t lr, float * yy, int64_t ly) {
-            return bm192 ? launch_gemm<4, 2, 32, 192, true, true>(wtype, wb, N, K, K * 2, xh, M, bi, re, lr, yy, ly, glu,
-                                                                   mul, spl, stream)
-                         : launch_gemm<4, 2, 32, 256, true, true>(wtype, wb, N, K, K * 2, xh, M, bi, re, lr, yy, ly, glu,
-                                                                   mul, spl, stream);
-        };
-        if (spl.n > 1) {
-            int rc = wide(nullptr, nullptr, 0, nullptr, N);
-            if (rc != MMHIP_OK) {
-                return rc;
-            }
-            const int64_t nt = M * (N / 4);
-            const int64_t nb = (nt + 255) / 256;
-            hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned) (nb < 16384 ? nb : 16384)), dim3(256), 0, stream,
-                               (const float *) spl.part, spl.n, M, N, bias, res, ldr, y, ldy);
-            return check_launch("mul_mat gemm: split-K reduce");
-        }
-        if (tiles256 >= 256 || (mul.n > 0 && tiles256 >= 128)) {
-            return wide(bias, res, ldr, y, ldy);
-        }
-        return launch_gemm<4, 2, 32, 64, true>(wtype, wb, N, K, K * 2, xh, M, bias, res, ldr, y, ldy, glu, mul, spl,
-                                               stream);
+                       const GemmMulti & mul, const GemmSplit & spl, hipStream_t stream) {
+    const bool   wh    = wtype == TYPE_F16 || wtype == TYPE_BF16;
+    const bool   split = spl.n > 1;
+    const double steps = (double) K / 64 / spl.n;
+    const double r256  = (double) (((N + 255) / 256 * ((M + 255) / 256) * spl.n + 255) / 256);
+    const double t256  = 5.0 + (split ? 6.0 : 0.0) + r256 * steps * (wh ? 2.1 : 2.3);
+    const double t64   = split ? 1e30 : 4.0 + steps * (0.3 + 0.0018 * (double) ((N + 127) / 128 * ((M + 63) / 64)));
+    int          bm    = 0;
+    const double tp    = gemm_p_takes(wtype, N, K, rs, spl.n) ? gemm_p_us(wtype, N, K, M, spl.n, bm) : 1e30;
+    const float * bi   = split ? nullptr : bias;
+    const float * re   = split ? nullptr : res;
+    float *       yy   = split ? nullptr : y;
+    const int64_t lr = split ? 0 : ldr, ly = split ? N : ldy;
+    int           rc;
+    if (tp < t256 && (!wh || tp < t64)) {
+        rc = gemm_p(bm, wtype, wb, N, K, rs, xh, M, bi, re, lr, yy, ly, glu, mul, spl, stream);
+    } else if (wh) {
+        rc = t256 < t64 ? launch_gemm<4, 2, 32, 256, true, true>(wtype, wb, N, K, rs, xh, M, bi, re, lr, yy, ly, glu, mul,
+                                                                 spl, stream)
+                        : launch_gemm<4, 2, 32, 64, true>(wtype, wb, N, K, rs, xh, M, bi, re, lr, yy, ly, glu, mul, spl,
+                                                          stream);
+    } else if (split || K % 256 == 0 || (N + 255) / 256 * ((M + 255) / 256) >= 256) {
+        rc = launch_gemm<8, 2, 64>(wtype, wb, N, K, rs, xh, M, bi, re, lr, yy, ly, glu, mul, spl, stream);
+    } else {
+        // Q8_0 rows of a width that is no multiple of 256, few tiles: 64
+        // tokens x 128 rows, three workgroups a CU
+        rc = launch_gemm<4, 2, 64, 64>(wtype, wb, N, K, rs, xh, M, bi, re, lr, yy, ly, glu, mul, spl, stream);
     }
-    if (spl.n > 1) {
-        // 256 x 256 tiles over K parts, then the ordered reduction with the ADDs
-        const GemmSplit sp = spl;
-        int rc = launch_gemm<8, 2, 64>(wtype, wb, N, K, rs, xh, M, nullptr, nullptr, 0, nullptr, N, glu, mul, sp, stream);
-        if (rc != MMHIP_OK) {
-            return rc;
-        }
-        const int64_t nt = M * (N / 4);
-        const int64_t nb = (nt + 255) / 256;
-        hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned) (nb < 16384 ? nb : 16384)), dim3(256), 0, stream,
-                           (const float *) spl.part, spl.n, M, N, bias, res, ldr, y, ldy);
-        return check_launch("mul_mat gemm: split-K reduce");
-    }
-    // several weight matrices in one launch: 256 x 256 tiles once they fill
-    // half the CUs (the DiT's q / k / v: 144 tiles), where three launches of
-    // small tiles ran at half the MFMA rate
-    if (tiles256 >= 256 || (mul.n > 0 && tiles256 >= 128)) {
-        return launch_gemm<8, 2, 64>(wtype, wb, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
-    }
-    // small grids (the DiT's 2048-row projections at 1380 tokens: 176 tiles of
-    // 128 x 128): 64-token x 128-row tiles, twice the workgroups, three per CU
-    // in LDS (a 128-wide K step on 128 x 128 tiles: 2.6 % slower per DiT block;
-    // 32 x 128 and 128 x 256 tiles: 1 % and 25 % slower)
-    return launch_gemm<4, 2, 64, 64>(wtype, wb, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+    return rc != MMHIP_OK || !split ? rc : splitk_reduce(spl, M, N, bias, res, ldr, y, ldy, stream);
 }
 
 // K parts for a shape: few 256 x 256 tiles (under half the CUs) and a long
@@ -1123,6 +932,10 @@ int gemm_q_h(int wtype, const void * W, int64_t N, int64_t K, int64_t rs, const 
     }
     const GemmGlu   none{};
     const GemmMulti single{};
+    if (gemm_sk_takes(wtype, mul ? mul->Nper : N, K, rs, M)) {
+        return gemm_sk(wtype, (const uint8_t *) W, N, K, rs, (const _Float16 *) xh, M, bias, res, ldr, y, ldy,
+                       glu ? *glu : none, mul ? *mul : single, stream);
+    }
     GemmSplit       spl;
     if (!glu && !mul && split_ws && split_ws_bytes >= gemm_split_bytes(N, K, M) && ((uintptr_t) split_ws) % 16 == 0) {
         spl.n    = gemm_split(N, K, M);
@@ -1145,8 +958,8 @@ int gemm_q_h(int wtype, const void * W, int64_t N, int64_t K, int64_t rs, const 
     } else {
         wh = f16_weights(W, N, K);
     }
-    return gemm_launch(wtype, (const uint8_t *) (wh ? wh : W), N, K, rs, (const _Float16 *) xh, M, bias, res, ldr, y,
-                       ldy, glu ? *glu : none, mf, spl, stream, wh != nullptr);
+    return gemm_launch(wh ? TYPE_F16 : wtype, (const uint8_t *) (wh ? wh : W), N, K, wh ? 2 * K : rs,
+                       (const _Float16 *) xh, M, bias, res, ldr, y, ldy, glu ? *glu : none, mf, spl, stream);
 }
 
 int convert_act_f16(const float * x, int64_t ldx, int64_t K, int64_t M, void * xh, hipStream_t stream) {
@@ -1175,6 +988,11 @@ int gemm_q(int wtype, const void * W, int64_t N, int64_t K, int64_t rs, const fl
     int           rc  = MMHIP_OK;
     const GemmGlu   none{};
     const GemmMulti single{};
+    if (gemm_sk_takes(wtype, N, K, rs, M)) {
+        rc = convert_act_f16(x, ldx, K, M, xh, stream);
+        return rc != MMHIP_OK ? rc : gemm_sk(wtype, (const uint8_t *) W, N, K, rs, xh, M, bias, res, ldr, y, ldy,
+                                             glu ? *glu : none, single, stream);
+    }
     GemmSplit       spl;
     // workspace: the f16 activations, [the f16 weights,] [the partial sums]
     const size_t    xo  = (need + 255) / 256 * 256;
@@ -1221,8 +1039,9 @@ int gemm_q(int wtype, const void * W, int64_t N, int64_t K, int64_t rs, const fl
             wb = (const uint8_t *) whp;
         }
     }
-    return gemm_launch(wtype, wb, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu ? *glu : none, single, spl, stream,
-                       wh || reg);
+    const bool w16 = wh || reg;
+    return gemm_launch(w16 ? TYPE_F16 : wtype, wb, N, K, w16 ? 2 * K : rs, xh, M, bias, res, ldr, y, ldy,
+                       glu ? *glu : none, single, spl, stream);
 }
 
 // BF16 weights at token counts: rows rs bytes apart read in place by the
@@ -1260,21 +1079,8 @@ int gemm_bf16(const void * W, int64_t N, int64_t K, int64_t rs, const float * x,
     const GemmGlu   none{};
     const GemmMulti single{};
     const GemmSplit one{};
-    const uint8_t * wb       = (const uint8_t *) W;
-    const auto *    xb       = (const _Float16 *) ws;  // 16-bit patterns
-    const int64_t   tiles256 = ((N + 255) / 256) * ((M + 255) / 256);
-    if (tiles256 >= 256) {
-        // 192-token tiles where they take fewer rounds by work (gemm_launch's rule)
-        const int64_t nn = (N + 255) / 256;
-        if (3 * ((nn * ((M + 191) / 192) + 255) / 256) < 4 * ((tiles256 + 255) / 256)) {
-            return launch_gemm<4, 2, 32, 192, true, true>(TYPE_BF16, wb, N, K, rs, xb, M, nullptr, nullptr, 0, y, ldy,
-                                                          none, single, one, stream);
-        }
-        return launch_gemm<4, 2, 32, 256, true, true>(TYPE_BF16, wb, N, K, rs, xb, M, nullptr, nullptr, 0, y, ldy, none,
-                                                      single, one, stream);
-    }
-    return launch_gemm<4, 2, 32, 64, true>(TYPE_BF16, wb, N, K, rs, xb, M, nullptr, nullptr, 0, y, ldy, none, single,
-                                           one, stream);
+    return gemm_launch(TYPE_BF16, (const uint8_t *) W, N, K, rs, (const _Float16 *) ws /* 16-bit patterns */, M, nullptr,
+                       nullptr, 0, y, ldy, none, single, one, stream);
 }
 
 // F32 weights at token counts (the DiT's k = 1 convs, src/dit.h:258 and

@@ -1,0 +1,397 @@
+// k_gemm_common.h - what the MFMA GEMMs of MUL_MAT share: the matrix
+// instructions, the LDS tile layout, the dequantising row loaders and the
+// epilogue.
+#pragma once
+
+#include <type_traits>
+
+#include "mmhip_device.h"
+#include "mmhip_internal.h"
+
+namespace mmhip {
+
+__device__ __forceinline__ float16_t gm_mfma(half8_t a, half8_t b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// The same product on bf16 operands (carried as 16-bit patterns in half8_t):
+// bf16 x bf16 products are exact in f32 and accumulate in f32.
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ float16_t gm_mfma_bf16(half8_t a, half8_t b, float16_t c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c,
+                                                   0, 0, 0);
+}
+
+// Tiles in LDS are unpadded rows of 64 halves (8 chunks of 16 bytes) with
+// chunk c of row r stored at chunk c ^ (r & 7): the 32 rows an MFMA operand
+// read touches then spread over all banks.
+template <int BK>
+__device__ __forceinline__ int swz(int r, int c) {
+    return r * BK + 8 * (c ^ (r & 7));
+}
+
+// ---------------------------------------------------------------------
+// Quantised rows read 64 columns at a time by four lanes (g = 0..3), C = the
+// step's place (0..3) in its 256 columns.  A lane's two operands P = 0, 1 are
+// eight consecutive columns each, at 16-byte chunk qr_chunk<WT>(g, P) of the
+// step's f16 row.  The values are the GGUF definitions' f32 results rounded
+// once to f16 (w_dequant in k_gemm.hip has the same, value for value):
+//   Q8_0      d * q as a packed f16 product: q is exact in f16, so the product
+//             is the exact one rounded once, as the f32 product's rounding is
+//   Q4_K/Q5_K d1 * q - m1 as one fma: d1 = d * sc and d1 * q are exact in f32
+//             (at most 22 bits), so the fma rounds where the difference does
+//   Q6_K      ds * (q - 32) as fma(q, ds, -32 ds): 32 ds is exact, so the fma
+//             rounds the exact product once, as the product does
+// QRow holds the quants (Q6_K: of two steps, one 128-column half, so it is
+// loaded at even C only), QScale what a row's 256 columns share; both are
+// loaded at row + ro, the pointer uniform and ro per lane.  k256: the first
+// of the 256 columns.
+typedef int      int2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t uint3_t __attribute__((ext_vector_type(3)));
+typedef float    float2_t __attribute__((ext_vector_type(2)));
+
+template <int WT> __device__ __forceinline__ int qr_chunk(int g, int p) {
+    return WT == TYPE_Q8_0 ? 2 * g + p : 4 * p + g;
+}
+
+// f((float) byte) for the four bytes of x, in f32, rounded to f16 by the
+// packed conversion
+template <class F> __device__ __forceinline__ void qr_bytes(uint32_t x, half8_t & o, int at, F f) {
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const float2_t v = { f((float) ((x >> (8 * i)) & 0xff)), f((float) ((x >> (8 * i + 8)) & 0xff)) };
+        const half2_t  h = __builtin_convertvector(v, half2_t);
+        o[at + i]        = h[0];
+        o[at + i + 1]    = h[1];
+    }
+}
+
+// Four Q8_0 quants times the f16 scale pair dd
+__device__ __forceinline__ void qr_q8(uint32_t q, half2_t dd, half8_t & o, int at) {
+    const half2_t  off = { (_Float16) 1152.0f, (_Float16) 1152.0f };
+    const uint32_t u   = q ^ 0x80808080u;  // q + 128
+    // 0x6400 | byte is the f16 1024 + byte
+    const half2_t a = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u));
+    const half2_t b = __builtin_bit_cast(half2_t, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u));
+    const half2_t x = (a - off) * dd, y = (b - off) * dd;
+    o[at]           = x[0];
+    o[at + 1]       = x[1];
+    o[at + 2]       = y[0];
+    o[at + 3]       = y[1];
+}
+
+// Scale and min of sub-block J (0..7) of a Q4_K / Q5_K super-block from its
+// twelve packed bytes
+template <int J> __device__ __forceinline__ void qr_scale_min(const uint3_t & s, float & sc, float & mn) {
+    constexpr int b = 8 * (J & 3);
+    if constexpr (J < 4) {
+        sc = (float) ((s[0] >> b) & 63);
+        mn = (float) ((s[1] >> b) & 63);
+    } else {
+        sc = (float) (((s[2] >> b) & 15) | (((s[0] >> (b + 6)) & 3) << 4));
+        mn = (float) (((s[2] >> (b + 4)) & 15) | (((s[1] >> (b + 6)) & 3) << 4));
+    }
+}
+
+template <int WT> struct QRow;
+template <int WT> struct QScale;
+
+template <> struct QRow<TYPE_Q8_0> {
+    int4_t q;
+    template <int C> __device__ __forceinline__ void load(const uint8_t * row, uint32_t ro, int64_t, int k256, int g) {
+        q = *(const int4_t *) (row + k256 + 64 * C + (ro + 16u * g));
+    }
+};
+template <> struct QScale<TYPE_Q8_0> {
+    int4_t d;  // eight f16 scales
+    __device__ __forceinline__ void load(const uint8_t * row, uint32_t ro, int64_t K, int k256, int) {
+        d = *(const int4_t *) (row + K + (k256 >> 4) + ro);
+    }
+};
+
+template <int WT> struct QRowK45 {
+    int2_t q;
+    template <int C> __device__ __forceinline__ void load(const uint8_t * row, uint32_t ro, int64_t, int k256, int g) {
+        q = *(const int2_t *) (row + (k256 >> 1) + 32 * C + (ro + 8u * g));
+    }
+};
+template <int WT> struct QScaleK45 {
+    uint3_t  s;
+    uint32_t dm;
+    int2_t   h;  // Q5_K: the fifth bits of this lane's columns in all four steps
+    __device__ __forceinline__ void load(const uint8_t * row, uint32_t ro, int64_t K, int k256, int g) {
+        const int64_t qh = WT == TYPE_Q5_K ? K / 8 : 0;
+        const int     sb = k256 >> 8;
+        __builtin_memcpy(&s, row + K / 2 + qh + 12 * sb + ro, 12);
+        dm = *(const uint32_t *) (row + K / 2 + qh + 12 * (K / 256) + 4 * sb + ro);
+        if constexpr (WT == TYPE_Q5_K) {
+            h = *(const int2_t *) (row + K / 2 + 32 * sb + (ro + 8u * g));
+        }
+    }
+};
+template <> struct QRow<TYPE_Q4_K> : QRowK45<TYPE_Q4_K> {};
+template <> struct QRow<TYPE_Q5_K> : QRowK45<TYPE_Q5_K> {};
+template <> struct QScale<TYPE_Q4_K> : QScaleK45<TYPE_Q4_K> {};
+template <> struct QScale<TYPE_Q5_K> : QScaleK45<TYPE_Q5_K> {};
+
+template <> struct QRow<TYPE_Q6_K> {
+    int2_t la, lb, h;
+    template <int C> __device__ __forceinline__ void load(const uint8_t * row, uint32_t ro, int64_t K, int k256, int g) {
+        const uint8_t * p = row + (k256 >> 1) + 64 * (C >> 1);
+        la = *(const int2_t *) (p + (ro + 8u * g));
+        lb = *(const int2_t *) (p + 32 + (ro + 8u * g));
+        h  = *(const int2_t *) (row + K / 2 + (k256 >> 2) + 32 * (C >> 1) + (ro + 8u * g));
+    }
+};
+template <> struct QScale<TYPE_Q6_K> {
+    int4_t   sc;  // sixteen int8 scales
+    uint16_t d;
+    __device__ __forceinline__ void load(const uint8_t * row, uint32_t ro, int64_t K, int k256, int) {
+        sc = *(const int4_t *) (row + K / 2 + K / 4 + (k256 >> 4) + ro);
+        d  = *(const uint16_t *) (row + K / 2 + K / 4 + K / 16 + (k256 >> 7) + ro);
+    }
+};
+
+template <int WT, int P, int C>
+__device__ __forceinline__ half8_t qr_operand(const QRow<WT> & r, const QScale<WT> & s, int g) {
+    half8_t o;
+    if constexpr (WT == TYPE_Q8_0) {
+        const _Float16 d  = __builtin_bit_cast(_Float16, (uint16_t) ((uint32_t) s.d[C] >> (16 * (g >> 1))));
+        const half2_t  dd = { d, d };
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            qr_q8((uint32_t) r.q[2 * P + w], dd, o, 4 * w);
+        }
+    } else if constexpr (WT == TYPE_Q6_K) {
+        constexpr int t  = C & 1;  // quarters 2t (P = 0) and 2t + 1 (P = 1) of the half
+        const float   ds = h2f(s.d) * (float) (int8_t) ((uint32_t) s.sc[C] >> (16 * P + 8 * (g >> 1)));
+        const float   off = -32.0f * ds;
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            const uint32_t l = (uint32_t) (P ? r.lb[w] : r.la[w]) >> (4 * t);
+            constexpr int  b = 4 * t + 2 * P;
+            const uint32_t v = (uint32_t) r.h[w];
+            const uint32_t x = (l & 0x0f0f0f0fu) | ((b <= 4 ? v << (4 - b) : v >> (b - 4)) & 0x30303030u);
+            qr_bytes(x, o, 4 * w, [&](float q) { return __builtin_fmaf(q, ds, off); });
+        }
+    } else {
+        float sc, mn;
+        qr_scale_min<2 * C + P>(s.s, sc, mn);
+        const float d1 = h2f((uint16_t) (s.dm & 0xffff)) * sc, m1 = h2f((uint16_t) (s.dm >> 16)) * mn;
+#pragma unroll
+        for (int w = 0; w < 2; w++) {
+            uint32_t x = ((uint32_t) r.q[w] >> (4 * P)) & 0x0f0f0f0fu;
+            if constexpr (WT == TYPE_Q5_K) {
+                constexpr int  b = 2 * C + P;
+                const uint32_t v = (uint32_t) s.h[w];
+                x |= (b <= 4 ? v << (4 - b) : v >> (b - 4)) & 0x10101010u;
+            }
+            qr_bytes(x, o, 4 * w, [&](float v) { return __builtin_fmaf(v, d1, -m1); });
+        }
+    }
+    return o;
+}
+
+// ---------------------------------------------------------------------
+// A workgroup's tile: first token, first weight row, K part.  Consecutive work
+// items (one XCD, one L2) share the operand that is re-read most: the weight
+// tile when there are more weight tiles than token tiles (its token tiles run
+// together), else the activation tiles, in groups of GM_GROUP token tiles
+// with the token tile fastest, so that the workgroups running together on an
+// XCD cover a block of GM_GROUP token tiles by several weight tiles and each
+// weight tile is fetched once per group rather than once per token tile.
+// Split-K: work items (part, tile), the parts of one tile n_base apart.
+constexpr int GM_GROUP = 4;
+
+__device__ __forceinline__ void gm_tile(int64_t n_ntiles, int64_t n_tiles, int parts, int bm, int bt, int64_t & m0,
+                                        int64_t & n0, int & kpart) {
+    const int64_t n_base = n_tiles / parts;
+    const int64_t lin    = xcd_remap(blockIdx.x, n_tiles);
+    kpart                = (int) (lin / n_base);
+    const int64_t work   = lin % n_base;
+    const int64_t n_mt   = n_base / n_ntiles;
+    if (n_ntiles > n_mt) {
+        m0 = work % n_mt * bm;
+        n0 = work / n_mt * bt;
+    } else {
+        const int64_t gsz = (int64_t) GM_GROUP * n_ntiles;
+        const int64_t g   = work / gsz, r = work % gsz;
+        const int64_t gw  = min((int64_t) GM_GROUP, n_mt - g * GM_GROUP);
+        m0                = (g * GM_GROUP + r % gw) * bm;
+        n0                = r / gw * bt;
+    }
+}
+
+// ---------------------------------------------------------------------
+// Epilogue of the tile kernels: the accumulators of a BM x BT tile held by
+// WM x WN waves of MB x NB blocks of 32 x 32.
+template <int MB, int NB, int BM, int BT, int WM, int WN, bool GLU>
+__device__ __forceinline__ void gm_epilogue(const float16_t (&acc)[MB][NB], int64_t m0, int64_t n0, int64_t N, int64_t M,
+                                            int wave, int lane, const float * __restrict__ bias, const float * res,
+                                            int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+                                            const GemmSplit & spl, int kpart) {
+#pragma clang fp contract(off)
+    const int wm = wave / WN, wn = wave % WN, lq = lane & 31, hh = lane >> 5;
+    // C[i = token][j = weight row]: lane holds row j = lq, tokens 8(r/4) + 4hh + r%4.
+    // Each epilogue runs branch-free on whole tiles (all but the last row and
+    // column of tiles): at the joins of per-element bounds branches the
+    // compiler waits for every store in flight, one wait per element.
+    const int64_t mw     = m0 + wm * (BM / WM) + 4 * hh;  // token of register 0 in block i = 0
+    const bool    full_m = m0 + BM <= M;
+    if constexpr (GLU) {
+        // pair p of this wave: value block 2p, gate block 2p + 1, SwiGLU column j
+        constexpr int NP = NB / 2;
+        int64_t       jp[NP];
+        float         bv[NP], bg[NP];
+#pragma unroll
+        for (int q = 0; q < NP; q++) {
+            jp[q]            = n0 / 2 + wn * (BT / WN / 2) + q * 32 + lq;
+            const bool    ok = jp[q] < glu.F;
+            const int64_t rv = glu.swapped ? glu.F + jp[q] : jp[q];  // value row
+            const int64_t rg = glu.swapped ? jp[q] : glu.F + jp[q];  // gate row
+            bv[q]            = bias && ok ? bias[rv] : 0.0f;
+            bg[q]            = bias && ok ? bias[rg] : 0.0f;
+        }
+        // the bias in registers before any store: a use behind a store's
+        // bounds branch would otherwise wait for all stores in flight
+        __builtin_amdgcn_s_waitcnt(0);
+        auto go = [&](auto full_c) {
+            constexpr bool FULL = decltype(full_c)::value;
+#pragma unroll
+            for (int q = 0; q < NP; q++) {
+                const int64_t j = jp[q];
+                if (j >= glu.F) {
+                    continue;
+                }
+#pragma unroll
+                for (int i = 0; i < MB; i++) {
+                    float o[16];
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        float v = acc[i][2 * q][r], g = acc[i][2 * q + 1][r];
+                        if (bias) {
+                            v = v + bv[q];
+                            g = g + bg[q];
+                        }
+                        const float silu = g / (1.0f + expf(-g));
+                        o[r]             = silu * v;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int64_t m = mw + i * 32 + 8 * (r / 4) + (r % 4);
+                        if (FULL || m < M) {
+                            if (glu.h) {
+                                glu.h[m * glu.F + j] = o[r];
+                            }
+                            if (glu.hh) {
+                                glu.hh[m * glu.F + j] = (_Float16) o[r];
+                            }
+                        }
+                    }
+                }
+            }
+        };
+        if (full_m) {
+            go(std::integral_constant<bool, true>{});
+        } else {
+            go(std::integral_constant<bool, false>{});
+        }
+        return;
+    }
+    const int64_t nl   = n0 + wn * (BT / WN) + lq;  // this lane's column in weight block 0
+    const bool    full = full_m && n0 + BT <= N;
+    if (spl.n > 1) {
+        // partial sums of this K part; the reduce kernel adds the ADDs
+        float * pp = spl.part + (int64_t) kpart * M * N;
+        auto    go = [&](auto full_c) {
+            constexpr bool FULL = decltype(full_c)::value;
+#pragma unroll
+            for (int i = 0; i < MB; i++) {
+#pragma unroll
+                for (int j = 0; j < NB; j++) {
+                    const int64_t n = nl + 32 * j;
+                    if (!FULL && n >= N) {
+                        continue;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const int64_t m = mw + i * 32 + 8 * (r / 4) + (r % 4);
+                        if (FULL || m < M) {
+                            pp[m * N + n] = acc[i][j][r];
+                        }
+                    }
+                }
+            }
+        };
+        if (full) {
+            go(std::integral_constant<bool, true>{});
+        } else {
+            go(std::integral_constant<bool, false>{});
+        }
+        return;
+    }
+    // Epilogue: the bias ADD, then the residual ADD, each rounded as its op.
+    // The bias is loaded once per column, and each 32 x 32 block's residual
+    // values are loaded before the previous block's stores are issued (loads
+    // and stores share one completion counter, so a load issued behind
+    // stores would wait for them too).  In place (res == y) every element is
+    // read before this thread writes it, and no other thread touches it.
+    float bn[NB];
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        bn[j] = bias && nl + 32 * j < N ? bias[nl + 32 * j] : 0.0f;
+    }
+    __builtin_amdgcn_s_waitcnt(0);  // the bias in registers before any store
+    auto go = [&](auto full_c) {
+        constexpr bool FULL = decltype(full_c)::value;
+        float          rv[16];
+        auto           rload = [&](int b) {
+            const int64_t n = nl + 32 * (b % NB);
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int64_t m = mw + (b / NB) * 32 + 8 * (r / 4) + (r % 4);
+                rv[r]           = FULL || (m < M && n < N) ? res[m * ldr + n] : 0.0f;
+            }
+        };
+        if (res) {
+            rload(0);
+        }
+#pragma unroll
+        for (int b = 0; b < MB * NB; b++) {
+            const int     i = b / NB, j = b % NB;
+            const int64_t n = nl + 32 * j;
+            float         v[16];
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                v[r] = bias ? acc[i][j][r] + bn[j] : acc[i][j][r];
+            }
+            if (res) {
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    v[r] = rv[r] + v[r];
+                }
+                if (b + 1 < MB * NB) {
+                    rload(b + 1);
+                }
+            }
+            if (!FULL && n >= N) {
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int64_t m = mw + i * 32 + 8 * (r / 4) + (r % 4);
+                if (FULL || m < M) {
+                    y[m * ldy + n] = v[r];
+                }
+            }
+        }
+    };
+    if (full) {
+        go(std::integral_constant<bool, true>{});
+    } else {
+        go(std::integral_constant<bool, false>{});
+    }
+}
+
+}  // namespace mmhip

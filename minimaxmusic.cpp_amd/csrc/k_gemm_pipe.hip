@@ -1,0 +1,387 @@
+// k_gemm_pipe.hip - MUL_MAT at token counts: the register-staged pipeline.
+//
+//   y[m, n] = sum_k x[m, k] * deq(W)[n, k]
+//
+// A workgroup of eight waves (two per SIMD) computes BM tokens x 256 weight
+// rows in steps of 64 columns.  The next steps' activations (f16) and weights
+// (quants as stored, or 16-bit rows) are loaded two steps ahead into
+// registers, coalesced (eight lanes a 128-byte row, four lanes a quantised
+// row's 64 columns, what 256 columns share loaded once for them), and written
+// to the other LDS stage while the current one is multiplied: the weights are
+// dequantised between the MFMAs, once per tile.  Each of the step's four
+// 16-column products has its operands read during the product before, so the
+// step has one barrier, placed before its last product.
+#include "k_gemm_common.h"
+
+namespace mmhip {
+
+constexpr int GP_NW = 8;
+constexpr int GP_BT = 256;
+constexpr int GP_BK = 64;
+
+template <int WT, int BM, bool GLU>
+__global__ __launch_bounds__(GP_NW * 64, 2) void k_gemm_p(const uint8_t * __restrict__ W, int64_t N, int64_t K,
+                                                           int64_t rs, const _Float16 * __restrict__ xh, int64_t M,
+                                                           const float * __restrict__ bias, const float * res,
+                                                           int64_t ldr, float * y, int64_t ldy, GemmGlu glu,
+                                                           GemmMulti mul, GemmSplit spl, int64_t n_ntiles,
+                                                           int64_t n_tiles) {
+#pragma clang fp contract(off)
+    constexpr bool WH  = WT == TYPE_F16 || WT == TYPE_BF16;  // 16-bit weight rows
+    constexpr int  T   = GP_NW * 64, WM = 2, WN = GP_NW / WM, BT = GP_BT, BK = GP_BK;
+    constexpr int  MB  = BM / WM / 32, NB = BT / WN / 32;
+    constexpr int  TIX = BM * BK, STG = TIX + BT * BK;  // halves: the activation tile, a stage
+    constexpr int  XL  = BM / (T / 8);                  // 16-byte activation loads per thread and step
+    constexpr int  WP  = BT / (T / (WH ? 8 : 4));       // passes over the weight rows
+    constexpr bool PAIR = WT == TYPE_Q6_K;              // loads two steps of weights at once
+    static_assert(XL >= 1 && MB >= 1 && (!GLU || NB % 2 == 0), "tile shape");
+    extern __shared__ __attribute__((aligned(16))) _Float16 g_lds[];
+
+    int64_t m0, n0;
+    int     kpart;
+    gm_tile(n_ntiles, n_tiles, spl.n, BM, BT, m0, n0, kpart);
+    if (mul.n > 0) {
+        // several weight matrices: this tile's rows come from matrix n0 / Nper
+        const int mi = (int) (n0 / mul.Nper);
+        n0 -= mi * mul.Nper;
+        W    = mul.W[mi];
+        y    = mul.y[mi];
+        ldy  = mul.ldy[mi];
+        bias = mul.bias[mi];
+        N    = mul.Nper;
+    }
+    const int tid  = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lane = tid & 63;
+    const int wm = wave / WN, wn = wave % WN, lq = lane & 31, hh = lane >> 5;
+
+    // the weight row of local tile row r, from the tile's first; rows past the
+    // end repeat a valid one and are never stored
+    auto wrow_of = [&](int r) -> int64_t {
+        if constexpr (GLU) {
+            // local row (wave block, value / gate, 32-row offset) -> SwiGLU column j
+            const int     wq = r / (BT / WN), blk = (r % (BT / WN)) / 32;
+            const int64_t j  = n0 / 2 + wq * (BT / WN / 2) + (blk / 2) * 32 + (r % 32);
+            return j >= glu.F ? 0 : (blk & 1) != (glu.swapped != 0) ? glu.F + j : j;  // from row 0
+        } else {
+            return n0 + r < N ? r : 0;
+        }
+    };
+    const int    xr_ = tid >> 3, xc = tid & 7;  // eight threads copy a row's 128 bytes
+    const char * xb  = (const char *) (xh + m0 * K);
+    uint32_t     xo[XL];
+#pragma unroll
+    for (int i = 0; i < XL; i++) {
+        const int r = xr_ + T / 8 * i;
+        xo[i]       = (uint32_t) ((m0 + r < M ? r : (int) (M - 1 - m0)) * 2 * (int) K + 16 * xc);
+    }
+    const int       wr_ = WH ? tid >> 3 : tid >> 2, g = tid & 3;
+    const uint8_t * wb = GLU ? W : W + n0 * rs;  // uniform: the loads add a 32-bit offset per lane
+    uint32_t        wo[WP];
+#pragma unroll
+    for (int i = 0; i < WP; i++) {
+        wo[i] = (uint32_t) (wrow_of(wr_ + (T / (WH ? 8 : 4)) * i) * rs + (WH ? 16 * xc : 0));
+    }
+    const int nk = (int) (K / BK / spl.n);  // K steps of this part
+    const int kb = kpart * nk * BK;         // its first column
+
+    struct Wq {
+        QRow<WH ? TYPE_Q8_0 : WT> r[WH ? 1 : WP];
+        int4_t                    h[WH ? WP : 1];
+    };
+    struct Ws {
+        QScale<WH ? TYPE_Q8_0 : WT> s[WH ? 1 : WP];
+    };
+    // activation slots: two steps ahead (one where 192 tokens leave no registers)
+    constexpr int XS = BM == 192 && !WH ? 1 : 2;
+    int4_t        xs[XS][XL];
+    Wq            wq[2];
+    // of the 256 columns of the step being written, and the next (Q6_K on 192
+    // tokens has no registers for both: loaded again once the last step used them)
+    constexpr bool ONE = PAIR && BM == 192;
+    Ws             sc, sn;
+    auto loadx = [&](int4_t (&x)[XL], int ks) {
+        const int k0 = kb + min(ks, nk - 1) * BK;
+#pragma unroll
+        for (int i = 0; i < XL; i++) {
+            x[i] = *(const int4_t *) (xb + 2 * k0 + xo[i]);
+        }
+    };
+    // weights of step ks4 + C (ks4 a multiple of four)
+    auto loadw = [&](Wq & w, int ks4, auto c_c) {
+        constexpr int C = decltype(c_c)::value;
+        if constexpr (WH) {
+            const int k0 = kb + min(ks4 + C, nk - 1) * BK;
+#pragma unroll
+            for (int i = 0; i < WP; i++) {
+                w.h[i] = *(const int4_t *) (wb + 2 * k0 + wo[i]);
+            }
+        } else {
+            const int k256 = kb + min(ks4, nk - 4) * BK;
+#pragma unroll
+            for (int i = 0; i < WP; i++) {
+                w.r[i].template load<C>(wb, wo[i], K, k256, g);
+            }
+        }
+    };
+    auto loads = [&](Ws & s, int ks4) {
+        if constexpr (!WH) {
+            const int k256 = kb + min(ks4, nk - 4) * BK;
+#pragma unroll
+            for (int i = 0; i < WP; i++) {
+                s.s[i].load(wb, wo[i], K, k256, g);
+            }
+        }
+    };
+    auto xwrite = [&](const int4_t (&x)[XL], int st) {
+#pragma unroll
+        for (int i = 0; i < XL; i++) {
+            *(int4_t *) &g_lds[st * STG + swz<BK>(xr_ + T / 8 * i, xc)] = x[i];
+        }
+    };
+    // half H of the passes
+    auto wwrite = [&](const Wq & w, const Ws & s, int st, auto c_c, auto h_c) {
+        constexpr int C = decltype(c_c)::value, H = decltype(h_c)::value;
+        _Float16 *    bw = g_lds + st * STG + TIX;
+#pragma unroll
+        for (int i = H * WP / 2; i < (H + 1) * WP / 2; i++) {
+            if constexpr (WH) {
+                *(int4_t *) &bw[swz<BK>(wr_ + T / 8 * i, xc)] = w.h[i];
+            } else {
+                const int r = wr_ + T / 4 * i;
+                *(half8_t *) &bw[swz<BK>(r, qr_chunk<WT>(g, 0))] = qr_operand<WT, 0, C>(w.r[i], s.s[i], g);
+                *(half8_t *) &bw[swz<BK>(r, qr_chunk<WT>(g, 1))] = qr_operand<WT, 1, C>(w.r[i], s.s[i], g);
+            }
+        }
+    };
+
+    float16_t acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; i++) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                acc[i][j][r] = 0.0f;
+            }
+        }
+    }
+    half8_t a[MB], b0[NB], b1[NB];
+    auto rda = [&](int st, int kk, int i) {
+        return *(const half8_t *) &g_lds[st * STG + swz<BK>(wm * (BM / WM) + i * 32 + lq, 2 * kk + hh)];
+    };
+    auto rdb = [&](int st, int kk, int j) {
+        return *(const half8_t *) &g_lds[st * STG + TIX + swz<BK>(wn * (BT / WN) + j * 32 + lq, 2 * kk + hh)];
+    };
+    // one 16-column product on operands b; the operands of product kk of
+    // stage st are read meanwhile: the weights into bn, the activations of a
+    // block in place once its MFMAs are issued
+    auto product = [&](const half8_t (&b)[NB], half8_t (&bn)[NB], int st, int kk) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            bn[j] = rdb(st, kk, j);
+        }
+#pragma unroll
+        for (int i = 0; i < MB; i++) {
+#pragma unroll
+            for (int j = 0; j < NB; j++) {
+                if constexpr (WT == TYPE_BF16) {
+                    acc[i][j] = gm_mfma_bf16(a[i], b[j], acc[i][j]);
+                } else {
+                    acc[i][j] = gm_mfma(a[i], b[j], acc[i][j]);
+                }
+            }
+            a[i] = rda(st, kk, i);
+        }
+    };
+    // that order, with the phase's LDS writes, loads and dequantisation spread
+    // between the MFMAs
+    auto spread = [&]() {
+#pragma unroll
+        for (int i = 0; i < MB * NB; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+            if (i < NB) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read: b
+            }
+            if (i % NB == NB - 1) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a
+            }
+            __builtin_amdgcn_sched_group_barrier(0x002, 8, 0);                // VALU
+            __builtin_amdgcn_sched_group_barrier(0x200, 4 / MB, 0);           // LDS write
+            __builtin_amdgcn_sched_group_barrier(0x020, MB >= 3 ? 1 : 2, 0);  // load
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // only this wave's LDS accesses: the loads in flight stay so
+    auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+
+    // step ks on stage ks & 1, U = ks & 3: multiplies it, writes step ks + 1
+    // (place C of its 256 columns) to the other stage and loads step ks + 3
+    auto step = [&](auto u_c, int ks) {
+        using std::integral_constant;
+        constexpr int U = decltype(u_c)::value, C = (U + 1) & 3, ST = U & 1;
+        constexpr int SLOT = PAIR ? C >> 1 : C & 1, XSLOT = C % XS;
+        if constexpr (C == 0 && !ONE) {
+            sc = sn;
+            loads(sn, ks + 5);
+        }
+        product(b0, b1, ST, 1);
+        wwrite(wq[SLOT], sc, ST ^ 1, integral_constant<int, C>{}, integral_constant<int, 0>{});
+        spread();
+        product(b1, b0, ST, 2);
+        xwrite(xs[XSLOT], ST ^ 1);
+        wwrite(wq[SLOT], sc, ST ^ 1, integral_constant<int, C>{}, integral_constant<int, 1>{});
+        loadx(xs[XSLOT], ks + 1 + XS);
+        spread();
+        product(b0, b1, ST, 3);
+        if constexpr (C == 3 && ONE) {
+            loads(sc, ks + 2);
+        }
+        if constexpr (!PAIR) {
+            loadw(wq[SLOT], ks + 1 - C + (C + 2) / 4 * 4, integral_constant<int, (C + 2) & 3>{});
+        } else if constexpr (C & 1) {
+            loadw(wq[SLOT], ks + 1 - C + 4, integral_constant<int, C>{});
+        }
+        spread();
+        lds_barrier();
+        product(b1, b0, ST ^ 1, 0);
+        spread();
+    };
+    using std::integral_constant;
+    loads(sc, 0);
+    loadw(wq[0], 0, integral_constant<int, 0>{});
+    loadx(xs[0], 0);
+    if constexpr (PAIR) {
+        loadw(wq[1], 0, integral_constant<int, 2>{});
+    } else {
+        loadw(wq[1], 0, integral_constant<int, 1>{});
+    }
+    if constexpr (XS > 1) {
+        loadx(xs[1], 1);
+    }
+    if constexpr (!ONE) {
+        loads(sn, 4);
+    }
+    wwrite(wq[0], sc, 0, integral_constant<int, 0>{}, integral_constant<int, 0>{});
+    wwrite(wq[0], sc, 0, integral_constant<int, 0>{}, integral_constant<int, 1>{});
+    xwrite(xs[0], 0);
+    loadx(xs[0], XS);
+    if constexpr (!PAIR) {
+        loadw(wq[0], 0, integral_constant<int, 2>{});
+    }
+    lds_barrier();
+#pragma unroll
+    for (int i = 0; i < MB; i++) {
+        a[i] = rda(0, 0, i);
+    }
+#pragma unroll
+    for (int j = 0; j < NB; j++) {
+        b0[j] = rdb(0, 0, j);
+    }
+    int ks = 0;
+    for (; ks + 4 <= nk; ks += 4) {
+        step(integral_constant<int, 0>{}, ks);
+        step(integral_constant<int, 1>{}, ks + 1);
+        step(integral_constant<int, 2>{}, ks + 2);
+        step(integral_constant<int, 3>{}, ks + 3);
+    }
+    if constexpr (WH) {
+        // 16-bit rows: any number of steps
+        if (ks < nk) {
+            step(integral_constant<int, 0>{}, ks);
+        }
+        if (ks + 1 < nk) {
+            step(integral_constant<int, 1>{}, ks + 1);
+        }
+        if (ks + 2 < nk) {
+            step(integral_constant<int, 2>{}, ks + 2);
+        }
+    }
+    gm_epilogue<MB, NB, BM, BT, WM, WN, GLU>(acc, m0, n0, N, M, wave, lane, bias, res, ldr, y, ldy, glu, spl, kpart);
+}
+
+// The tile of fewest microseconds by the times measured: a step of 64 columns
+// takes c0 on an otherwise idle chip and c0 + c1 with all CUs at it, more
+// where the weights are too many to stay in the memory-side cache; 5 us of
+// launch, prologue and epilogue, 6 of split-K reduction.  (Q8_0 and f16 rows;
+// Q4_K to Q6_K take up to a quarter more on each tile alike.)
+double gemm_p_us(int wtype, int64_t N, int64_t K, int64_t M, int parts, int & bm) {
+    (void) wtype;
+    const struct { int bm; double c0, c1, far; } tile[3] = { { 64, 0.64, 0.20, 0.30 },
+                                                             { 128, 0.85, 0.30, 0.35 },
+                                                             { 192, 1.10, 0.65, 0.05 } };
+    const double steps = (double) K / GP_BK / parts;
+    const bool   far   = N * K > 64000000;
+    double       best  = 1e30;
+    for (const auto & t : tile) {
+        const int64_t tiles = (N + GP_BT - 1) / GP_BT * ((M + t.bm - 1) / t.bm) * parts, rem = tiles % 256;
+        const double  c0    = t.c0 + (far ? t.far : 0.0);
+        const double  us    = 5.0 + (parts > 1 ? 6.0 : 0.0) +
+                          steps * ((double) (tiles / 256) * (c0 + t.c1) + (rem ? c0 + t.c1 * (double) rem / 256.0 : 0.0));
+        if (us < best) {
+            best = us;
+            bm   = t.bm;
+        }
+    }
+    return best;
+}
+
+// Quantised rows come 256 columns at a time, also in each K part; 16-bit rows
+// in steps of 64.
+bool gemm_p_takes(int wtype, int64_t N, int64_t K, int64_t rs, int parts) {
+    const bool wh = wtype == TYPE_F16 || wtype == TYPE_BF16;
+    return K % ((wh ? GP_BK : 256) * parts) == 0 && K < (1 << 22) && rs < (1 << 23) && N * rs < ((int64_t) 1 << 32);
+}
+
+template <int WT, int BM, bool GLU>
+static int gp_launch(const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+                     const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+                     const GemmMulti & mul, const GemmSplit & spl, hipStream_t stream) {
+    const int64_t n_nt = (N + GP_BT - 1) / GP_BT;
+    const int64_t n    = n_nt * ((M + BM - 1) / BM) * spl.n;
+    if (n > 0x7fffffff) {
+        return set_error(MMHIP_ERR_UNSUPPORTED, "mul_mat gemm: too many tiles");
+    }
+    constexpr size_t lds  = (size_t) 2 * (BM + GP_BT) * GP_BK * sizeof(_Float16);
+    auto             kern = k_gemm_p<WT, BM, GLU>;
+    if (!ensure_lds_limit((const void *) kern, lds)) {
+        return set_error(MMHIP_ERR_HIP, "mul_mat gemm: cannot raise LDS limit to %zu", lds);
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned) n), dim3(GP_NW * 64), lds, stream, W, N, K, rs, xh, M, bias, res, ldr, y,
+                       ldy, glu, mul, spl, n_nt, n);
+    return check_launch("mul_mat gemm");
+}
+
+template <int BM, bool GLU>
+static int gp_type(int wtype, const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+                   const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+                   const GemmMulti & mul, const GemmSplit & spl, hipStream_t stream) {
+    switch (wtype) {
+        case TYPE_F16: return gp_launch<TYPE_F16, BM, GLU>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+        case TYPE_Q8_0: return gp_launch<TYPE_Q8_0, BM, GLU>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+        case TYPE_Q4_K: return gp_launch<TYPE_Q4_K, BM, GLU>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+        case TYPE_Q5_K: return gp_launch<TYPE_Q5_K, BM, GLU>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+        case TYPE_Q6_K: return gp_launch<TYPE_Q6_K, BM, GLU>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+    }
+    if constexpr (!GLU) {
+        return gp_launch<TYPE_BF16, BM, false>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+    }
+    return set_error(MMHIP_ERR_UNSUPPORTED, "mul_mat gemm: weight type %d", wtype);
+}
+
+int gemm_p(int bm, int wtype, const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+           const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+           const GemmMulti & mul, const GemmSplit & spl, hipStream_t stream) {
+    auto go = [&](auto bm_c) {
+        constexpr int BM = decltype(bm_c)::value;
+        return glu.F > 0 ? gp_type<BM, true>(wtype, W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream)
+                         : gp_type<BM, false>(wtype, W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, spl, stream);
+    };
+    switch (bm) {
+        case 64: return go(std::integral_constant<int, 64>{});
+        case 128: return go(std::integral_constant<int, 128>{});
+        default: return go(std::integral_constant<int, 192>{});
+    }
+}
+
+}  // namespace mmhip

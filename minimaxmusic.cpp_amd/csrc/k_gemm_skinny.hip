@@ -1,0 +1,388 @@
+// k_gemm_skinny.hip - MUL_MAT at few tokens (17 .. GEMM_SK_MAX_M): the
+// quantised weights are streamed once, dequantised in registers straight into
+// MFMA operands.
+//
+//   y[m, n] = sum_k x[m, k] * deq(W)[n, k]
+//
+// What bounds it: the weight bytes (HBM); a tile GEMM at these token counts
+// leaves most CUs without a tile, multiplies padding and dequantises through
+// LDS.  One workgroup owns 16 * RG weight rows and up to 64 tokens over the
+// whole of K, its eight waves splitting K into contiguous ranges: a wave
+// loads its rows' quants, dequantises them (exactly as k_gemm_q does: f32
+// arithmetic, one rounding to f16) into the A operand of
+// v_mfma_f32_16x16x32_f16 and multiplies them with its own slice of the f16
+// activations, which it stages through a private piece of LDS (coalesced
+// 128-byte rows in, conflict-free 16-byte operands out), so the loop has no
+// barrier.  At the end the eight partial sums are added in wave order in LDS
+// and the epilogue (bias, residual, or the SwiGLU of value / gate rows) runs
+// on the sums: no workspace and no second launch, and the same sums for every
+// form of the call.
+#include "k_gemm_common.h"
+
+namespace mmhip {
+
+constexpr int SK_NW   = 8;    // waves: parts of K
+constexpr int SK_STEP = 64;   // columns a wave takes per step
+
+__device__ __forceinline__ float4_t sk_mfma(half8_t a, half8_t b, float4_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+
+// MB: 16-token blocks; RG: 16-row groups (GLU: the first half of them value
+// rows, the second the gate rows of the same columns).
+template <int WT, int MB, int RG, bool GLU>
+__global__ __launch_bounds__(SK_NW * 64, 2) void k_gemm_sk(const uint8_t * __restrict__ W, int64_t N, int64_t K,
+                                                            int64_t rs, const _Float16 * __restrict__ xh, int64_t M,
+                                                            const float * __restrict__ bias, const float * res,
+                                                            int64_t ldr, float * y, int64_t ldy, GemmGlu glu,
+                                                            GemmMulti mul, int n_mt, int64_t n_tiles) {
+#pragma clang fp contract(off)
+    constexpr int XI = 2 * MB;         // activation loads per lane per step
+    constexpr int MT = 16 * MB;        // tokens
+    constexpr int RW = GLU ? RG / 2 : RG;  // row groups of output columns
+    static_assert(!GLU || RG % 2 == 0, "tile shape");
+    extern __shared__ __attribute__((aligned(16))) _Float16 sk_lds[];
+
+    const int64_t lin = xcd_remap(blockIdx.x, n_tiles);
+    const int64_t m0  = (lin % n_mt) * MT;
+    int64_t       n0  = (lin / n_mt) * (16 * RW);
+    if (mul.n > 0) {
+        const int mi = (int) (n0 / mul.Nper);
+        n0 -= mi * mul.Nper;
+        W    = mul.W[mi];
+        y    = mul.y[mi];
+        ldy  = mul.ldy[mi];
+        bias = mul.bias[mi];
+        N    = mul.Nper;
+    }
+    const int     tid  = threadIdx.x;
+    const int     wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int     lane = tid & 63;
+    const int     li   = lane & 15;
+    const int     g    = lane >> 4;
+    const int64_t NC   = GLU ? glu.F : N;  // output columns
+
+    // row group base (uniform) and this lane's row inside it; rows past the
+    // end repeat the last one and are not stored
+    const uint8_t * wb[RG];
+    uint32_t        ro[RG];
+#pragma unroll
+    for (int q = 0; q < RG; q++) {
+        const int64_t c0 = n0 + 16 * (q % RW);
+        const int64_t cb = c0 < NC ? c0 : NC - 1;
+        const int64_t up = GLU && ((q >= RW) != (glu.swapped != 0)) ? glu.F : 0;
+        const int64_t left = NC - cb;
+        wb[q] = W + (cb + up) * rs;
+        ro[q] = (uint32_t) ((li < left ? li : left - 1) * rs);
+    }
+    const int    kw   = wave * (int) (K / SK_NW);  // this wave's columns
+    const int    ns   = (int) (K / SK_NW) / SK_STEP;
+    const char * xb   = (const char *) (xh + m0 * K + kw);
+    const int    mrem = (int) (M - m0 < MT ? M - m0 : MT);
+    uint32_t     xo[XI];
+#pragma unroll
+    for (int i = 0; i < XI; i++) {
+        const int r = 8 * i + (lane >> 3);
+        xo[i]       = (uint32_t) ((r < mrem ? r : mrem - 1) * 2 * (int) K + 16 * (lane & 7));
+    }
+    _Float16 * xs = sk_lds + wave * (MT * SK_STEP);
+    // chunk c of row r at c ^ (r & 7)
+    _Float16 * xw = xs + (lane >> 3) * SK_STEP + 8 * ((lane & 7) ^ (lane >> 3));
+
+    int4_t         xr[XI];
+    // weights are loaded two steps ahead; Q6_K rows two steps at once: slot 0
+    // the first pair of the four, slot 1 the second
+    constexpr bool PAIR = WT == TYPE_Q6_K;
+    QRow<WT>       wr[2][RG];
+    QScale<WT>     sc[RG], sn[RG];  // of these 256 columns and the next
+    float4_t       acc[RG][MB];
+#pragma unroll
+    for (int q = 0; q < RG; q++) {
+#pragma unroll
+        for (int j = 0; j < MB; j++) {
+            acc[q][j] = float4_t{ 0.0f, 0.0f, 0.0f, 0.0f };
+        }
+    }
+    auto loadx = [&](int4_t (&r)[XI], int s) {
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            r[i] = *(const int4_t *) (xb + 2 * SK_STEP * s + xo[i]);
+        }
+    };
+    auto loadw = [&](QRow<WT> (&r)[RG], int s4, auto c_c) {
+#pragma unroll
+        for (int q = 0; q < RG; q++) {
+            r[q].template load<decltype(c_c)::value>(wb[q], ro[q], K, kw + SK_STEP * s4, g);
+        }
+    };
+    auto loads = [&](QScale<WT> (&r)[RG], int s4) {
+#pragma unroll
+        for (int q = 0; q < RG; q++) {
+            r[q].load(wb[q], ro[q], K, kw + SK_STEP * s4, g);
+        }
+    };
+    auto half = [&](auto p_c, auto c_c, const QRow<WT> (&r)[RG]) {
+        constexpr int P = decltype(p_c)::value, C = decltype(c_c)::value;
+        half8_t       b[MB];
+#pragma unroll
+        for (int j = 0; j < MB; j++) {
+            b[j] = *(const half8_t *) (xs + (16 * j + li) * SK_STEP + 8 * (qr_chunk<WT>(g, P) ^ (li & 7)));
+        }
+#pragma unroll
+        for (int q = 0; q < RG; q++) {
+            const half8_t a = qr_operand<WT, P, C>(r[q], sc[q], g);
+#pragma unroll
+            for (int j = 0; j < MB; j++) {
+                acc[q][j] = sk_mfma(a, b[j], acc[q][j]);
+            }
+        }
+    };
+    auto step = [&](auto c_c, auto last_c, int s) {
+        constexpr int  C    = decltype(c_c)::value;
+        constexpr bool LAST = decltype(last_c)::value;  // the last four steps: load only what they use
+        // the other lanes' operand reads of the step before are done (one
+        // wave, LDS in order); the compiler must not move accesses over this
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            *(int4_t *) (xw + 8 * i * SK_STEP) = xr[i];
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        if constexpr (!LAST || C < 3) {
+            loadx(xr, s + 1);
+        }
+        if constexpr (!LAST && C == 0) {
+            loads(sn, s + 4);
+        }
+        constexpr int SLOT = PAIR ? C >> 1 : C & 1;
+        half(std::integral_constant<int, 0>{}, c_c, wr[SLOT]);
+        half(std::integral_constant<int, 1>{}, c_c, wr[SLOT]);
+        if constexpr (PAIR) {
+            if constexpr (!LAST && C % 2 == 1) {
+                loadw(wr[SLOT], s - C + 4, c_c);
+            }
+        } else if constexpr (!LAST || C < 2) {
+            loadw(wr[SLOT], s - C + (C + 2) / 4 * 4, std::integral_constant<int, (C + 2) & 3>{});
+        }
+    };
+    auto four = [&](auto last_c, int s) {
+        step(std::integral_constant<int, 0>{}, last_c, s);
+        step(std::integral_constant<int, 1>{}, last_c, s + 1);
+        step(std::integral_constant<int, 2>{}, last_c, s + 2);
+        step(std::integral_constant<int, 3>{}, last_c, s + 3);
+        if constexpr (!decltype(last_c)::value) {
+#pragma unroll
+            for (int q = 0; q < RG; q++) {
+                sc[q] = sn[q];
+            }
+        }
+    };
+    loadx(xr, 0);
+    loads(sc, 0);
+    loadw(wr[0], 0, std::integral_constant<int, 0>{});
+    loadw(wr[1], 0, std::integral_constant<int, PAIR ? 2 : 1>{});
+    int s = 0;
+    for (; s + 4 < ns; s += 4) {
+        four(std::false_type{}, s);
+    }
+    four(std::true_type{}, s);
+
+    // D[i = weight row][j = token]: lane holds token li, rows 4g .. 4g + 3.
+    // The waves' sums of two row groups at a time meet in LDS (row quad q of
+    // token t at q ^ ((t >> 1) & 3): conflict-free 16-byte accesses).
+    float *   red   = (float *) sk_lds;
+    const int quad  = tid & 3, tok = (tid >> 2) % MT, sel = (tid >> 2) / MT;
+    auto      at    = [&](int q, int w, int t, int qd) { return (((q * SK_NW + w) * MT + t) * 4 + (qd ^ ((t >> 1) & 3))) * 4; };
+    auto      total = [&](int q) {
+        float4_t v = *(const float4_t *) (red + at(q, 0, tok, quad));
+#pragma unroll
+        for (int w = 1; w < SK_NW; w++) {
+            const float4_t u = *(const float4_t *) (red + at(q, w, tok, quad));
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                v[e] = v[e] + u[e];
+            }
+        }
+        return v;
+    };
+    auto put = [&](int q, int slot) {
+#pragma unroll
+        for (int j = 0; j < MB; j++) {
+            *(float4_t *) (red + at(slot, wave, 16 * j + li, g)) = acc[q][j];
+        }
+    };
+    const int64_t m = m0 + tok;
+    if constexpr (GLU) {
+#pragma unroll
+        for (int q = 0; q < RW; q++) {
+            __syncthreads();
+            put(q, 0);
+            put(q + RW, 1);
+            __syncthreads();
+            const int64_t j = n0 + 16 * q + 4 * quad;
+            if (sel == 0 && m < M) {
+                float4_t       v = total(0), gt = total(1);
+                const float *  bv = bias ? bias + (glu.swapped ? glu.F : 0) : nullptr;
+                const float *  bg = bias ? bias + (glu.swapped ? 0 : glu.F) : nullptr;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (j + e < glu.F) {
+                        if (bias) {
+                            v[e]  = v[e] + bv[j + e];
+                            gt[e] = gt[e] + bg[j + e];
+                        }
+                        const float silu = gt[e] / (1.0f + expf(-gt[e]));
+                        const float o    = silu * v[e];
+                        if (glu.h) {
+                            glu.h[m * glu.F + j + e] = o;
+                        }
+                        if (glu.hh) {
+                            glu.hh[m * glu.F + j + e] = (_Float16) o;
+                        }
+                    }
+                }
+            }
+        }
+    } else {
+        const bool vec = ldy % 4 == 0 && ((uintptr_t) y) % 16 == 0;
+#pragma unroll
+        for (int q = 0; q < RG; q += 2) {
+            __syncthreads();
+            put(q, 0);
+            if (q + 1 < RG) {
+                put(q + 1, 1);
+            }
+            __syncthreads();
+            const int64_t n = n0 + 16 * (q + sel) + 4 * quad;
+            if (sel < 2 && q + sel < RG && m < M && n < N) {
+                float4_t v = total(sel);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    if (n + e < N) {
+                        if (bias) {
+                            v[e] = v[e] + bias[n + e];
+                        }
+                        if (res) {
+                            v[e] = res[m * ldr + n + e] + v[e];
+                        }
+                    }
+                }
+                if (vec && n + 4 <= N) {
+                    *(float4_t *) (y + m * ldy + n) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        if (n + e < N) {
+                            y[m * ldy + n + e] = v[e];
+                        }
+                    }
+                }
+            }
+        }
+    }
+}
+
+// Rows a workgroup takes, in groups of 16: the fewest that leave no more
+// workgroups than CUs (a second workgroup of a CU adds its whole time:
+// 6144 x 4096 at 64 tokens 16.5 us on 192 workgroups of 32 rows, 22.4 on 384
+// of 16), at most 3 (48 rows on 24576 x 4096: 40.7 us, 32 rows 47.1, 64 rows,
+// which spill, 57.8).  Q6_K on more than 32 tokens spills at 3 (54.6 against
+// 47.9 us at 2).
+static int sk_groups(int wtype, int64_t N, int64_t M, int mb, bool two) {
+    const int64_t g16 = (N + 15) / 16 * ((M + 16 * mb - 1) / (16 * mb));
+    const int     top = two || (wtype == TYPE_Q6_K && mb > 2) ? 2 : 3;
+    return (int) (g16 <= 256 ? 1 : g16 <= 512 ? 2 : top);
+}
+
+// 16-token blocks of a tile: the fewest tiles of at most 64 tokens, each as
+// small as holds its share.
+static int sk_blocks(int64_t M) {
+    const int64_t n_mt = (M + 63) / 64;
+    const int64_t mb   = ((M + n_mt - 1) / n_mt + 15) / 16;
+    return mb < 2 ? 2 : (int) mb;
+}
+
+// Where the kernel is taken: K in whole 256-column blocks for each of the
+// eight waves, and either one tile of tokens (up to 64, where nothing else
+// comes near: 40 tokens x 4096 x 4096 Q8_0 9.2 us against 20 for the 64-token
+// pipeline tiles) or, up to GEMM_SK_MAX_M tokens, less time than the pipeline
+// would take, by the times measured for both (us).  The rule knows the type
+// and the sizes only, so every form of a call takes the same path.
+bool gemm_sk_takes(int wtype, int64_t N, int64_t K, int64_t rs, int64_t M) {
+    if (M > GEMM_SK_MAX_M || K % (256 * SK_NW) != 0 || K >= (1 << 23) || rs >= (1 << 24)) {
+        return false;
+    }
+    if (M <= 64) {
+        return true;
+    }
+    const int     mb = sk_blocks(M), rg = sk_groups(wtype, N, M, mb, false);
+    const int64_t wg = ((N + 16 * rg - 1) / (16 * rg)) * ((M + 16 * mb - 1) / (16 * mb));
+    const double  round[4] = { 0.0, 2.2, 3.0, 4.3 };  // a round of 256 workgroups, per 1024 columns
+    const double  t = 3.5 + (double) ((wg + 255) / 256) * (double) K / 1024.0 * round[rg];
+    int           bm;
+    return t < gemm_p_us(wtype, N, K, M, gemm_split(N, K, M), bm);
+}
+
+template <int WT, int MB, int RG, bool GLU>
+static int sk_launch(const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+                     const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+                     const GemmMulti & mul, hipStream_t stream) {
+    constexpr int MT    = 16 * MB;
+    const int64_t n_mt  = (M + MT - 1) / MT;
+    const int64_t per   = 16 * (GLU ? RG / 2 : RG);
+    const int64_t tiles = ((GLU ? glu.F : N) + per - 1) / per * n_mt;
+    if (tiles > 0x7fffffff) {
+        return set_error(MMHIP_ERR_UNSUPPORTED, "mul_mat gemm: too many tiles");
+    }
+    // the wave's activation slices, then two row groups of the waves' sums
+    constexpr size_t lds = (size_t) SK_NW * MT * SK_STEP * sizeof(_Float16);
+    static_assert(lds >= (size_t) 2 * SK_NW * MT * 16 * sizeof(float), "the sums fit the slices' space");
+    static_assert(lds <= 64 * 1024, "within the default LDS limit");
+    hipLaunchKernelGGL((k_gemm_sk<WT, MB, RG, GLU>), dim3((unsigned) tiles), dim3(SK_NW * 64), lds, stream, W, N, K, rs,
+                       xh, M, bias, res, ldr, y, ldy, glu, mul, (int) n_mt, tiles);
+    return check_launch("mul_mat gemm (few tokens)");
+}
+
+template <int WT, int MB>
+static int sk_rows(const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+                   const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+                   const GemmMulti & mul, hipStream_t stream) {
+    if (glu.F > 0) {
+        return sk_launch<WT, MB, 2, true>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+    }
+    // several matrices: 32 rows at most, so that no tile straddles two
+    switch (sk_groups(WT, N, M, MB, mul.n > 0)) {
+        case 1: return sk_launch<WT, MB, 1, false>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+        case 2: return sk_launch<WT, MB, 2, false>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+    }
+    if constexpr (WT != TYPE_Q6_K || MB <= 2) {
+        return sk_launch<WT, MB, 3, false>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+    }
+    return set_error(MMHIP_ERR_UNSUPPORTED, "mul_mat gemm: no tile for type %d", WT);
+}
+
+template <int WT>
+static int sk_tokens(const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+                     const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+                     const GemmMulti & mul, hipStream_t stream) {
+    switch (sk_blocks(M)) {
+        case 2: return sk_rows<WT, 2>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+        case 3: return sk_rows<WT, 3>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+        default: return sk_rows<WT, 4>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+    }
+}
+
+int gemm_sk(int wtype, const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+            const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+            const GemmMulti & mul, hipStream_t stream) {
+    switch (wtype) {
+        case TYPE_Q8_0: return sk_tokens<TYPE_Q8_0>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+        case TYPE_Q4_K: return sk_tokens<TYPE_Q4_K>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+        case TYPE_Q5_K: return sk_tokens<TYPE_Q5_K>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+        default: return sk_tokens<TYPE_Q6_K>(W, N, K, rs, xh, M, bias, res, ldr, y, ldy, glu, mul, stream);
+    }
+}
+
+}  // namespace mmhip

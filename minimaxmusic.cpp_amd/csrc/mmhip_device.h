@@ -63,6 +63,13 @@ __device__ __forceinline__ uint16_t f2h(float f) {
     return h;
 }
 
+// Consecutive work items go to one XCD (workgroups are dealt round-robin over
+// the 8 XCDs), so the workgroups sharing an activation tile share an L2.
+__device__ __forceinline__ int64_t xcd_remap(int64_t lin, int64_t total) {
+    const int64_t per = total / 8;
+    return lin >= per * 8 ? lin : (lin % 8) * per + lin / 8;
+}
+
 // Signed 4-byte dot product with int32 accumulate (v_dot4_i32_i8).
 __device__ __forceinline__ int dot4(int a, int b, int c) {
     return __builtin_amdgcn_sdot4(a, b, c, false);

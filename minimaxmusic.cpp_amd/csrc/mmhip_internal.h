@@ -109,6 +109,24 @@ struct GemmSplit {
     int     n    = 1;
     float * part = nullptr;
 };
+// MUL_MAT at few tokens (k_gemm_skinny.hip): the shapes it takes, in every
+// form of the call (N: the rows of one matrix; also where an f16 copy of the
+// weights is registered: it reads fewer bytes), and the call on f16
+// activations.
+constexpr int64_t GEMM_SK_MAX_M = 1024;
+bool gemm_sk_takes(int wtype, int64_t N, int64_t K, int64_t rs, int64_t M);
+int  gemm_sk(int wtype, const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+             const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+             const GemmMulti & mul, hipStream_t stream);
+// The register-staged pipeline (k_gemm_pipe.hip) on tiles of bm (64, 128 or
+// 192) tokens x 256 weight rows: quantised weights, or 16-bit rows (wtype F16
+// or BF16); with spl.n > 1 the parts' sums go to spl.part.  gemm_p_us: its
+// estimated time on the best tile, returned in bm.
+bool   gemm_p_takes(int wtype, int64_t N, int64_t K, int64_t rs, int parts);
+double gemm_p_us(int wtype, int64_t N, int64_t K, int64_t M, int parts, int & bm);
+int    gemm_p(int bm, int wtype, const uint8_t * W, int64_t N, int64_t K, int64_t rs, const _Float16 * xh, int64_t M,
+              const float * bias, const float * res, int64_t ldr, float * y, int64_t ldy, const GemmGlu & glu,
+              const GemmMulti & mul, const GemmSplit & spl, hipStream_t stream);
 // Parts the GEMM would split K into for this shape (1: no split), and the
 // bytes of partial sums that takes.
 int    gemm_split(int64_t N, int64_t K, int64_t M);

@@ -1,0 +1,146 @@
+"""GPU: MUL_MAT above 16 tokens at the edges of its kernels' tiles.
+
+The few-token kernel (16-row groups, 16-token blocks, K in eight parts) and
+the register-staged pipeline (64 / 128 / 192 tokens x 256 rows, with and
+without split K) against float64 products of the same operands rounded to f16
+(bf16): what remains is the order of the f32 sums, at most 2^-24 per addition
+on partial sums that grow like a random walk, so below 2^-24 sqrt(K) of the
+result's RMS; K <= 4096 gives 4e-6 on the relative RMS.  Outputs go to wider,
+NaN-filled rows, whose padding must stay as it is.  Every form of one product
+(bias, residual, SwiGLU, several matrices, f16 activations, a registered f16
+copy) takes the same path and gives the same sums."""
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+Q8_0, Q4_K, Q5_K, Q6_K = 8, 12, 13, 14
+
+
+def ptr(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def stream():
+    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+
+
+def weight(mm, pkg, t, N, K, seed):
+    """Rows padded to the 16 bytes the GEMMs' loads need."""
+    W = mm.QuantWeight.from_gguf(t, pkg.synth.gguf_blocks_torch(t, N, K, seed), N, K)
+    W.exact = W.dequantize()
+    pad = -W.row_bytes % 16
+    if pad:
+        W.data = torch.nn.functional.pad(W.data.view(N, W.row_bytes), (0, pad)).contiguous()
+        W.row_bytes += pad
+    return W
+
+
+def rel_rms(y, ref):
+    return ((y.double() - ref).norm() / ref.norm()).item()
+
+
+CASES = (
+    # few tokens: 1, 2 and 3 row groups, 2 to 4 token blocks and more tiles, row and token remainders
+    [(t, N, 2048, M) for t in (Q8_0, Q4_K, Q5_K, Q6_K) for N, M in ((100, 17), (4111, 33), (9000, 64), (250, 130))]
+    + [(Q8_0, 12500, 2048, 48), (Q6_K, 12500, 2048, 32), (Q6_K, 9000, 2048, 49), (Q5_K, 16, 4096, 63),
+       (Q4_K, 4096, 4096, 65), (Q8_0, 6144, 2048, 128)]
+    # pipeline tiles of 64, 128 and 192 tokens (no multiple of 2048 columns), one super-block of columns
+    + [(t, N, 768, M) for t in (Q8_0, Q4_K, Q5_K, Q6_K) for N, M in ((300, 65), (6000, 690), (6000, 1380))]
+    + [(Q6_K, 513, 256, 193), (Q8_0, 255, 256, 129), (Q4_K, 257, 1280, 191)]
+    # split K
+    + [(t, 1000, 3072 + 1024 * 2, 300) for t in (Q8_0, Q6_K)]
+    # columns that fill no 256: the 64 x 128 register-staged tiles
+    + [(Q8_0, 300, 320, 70)]
+)
+
+
+@pytest.mark.parametrize("t,N,K,M", CASES)
+def test_tile_edges(mm, pkg, t, N, K, M):
+    W = weight(mm, pkg, t, N, K, 9000 + N + M)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9100 + M)
+    x = torch.randn((M, K), device="cuda", generator=g)
+    bias = torch.randn(N, device="cuda", generator=g)
+    res = torch.randn((M, N), device="cuda", generator=g)
+    L = mm.load()
+    prod = x.half().double() @ W.exact.half().double().T
+    ref = prod + bias.double() + res.double()
+    for pad in (0, 3, 4):  # rows that are and are not 16-byte aligned
+        y = torch.full((M, N + pad), float("nan"), device="cuda")
+        need = L.mmhip_mul_mat_workspace(t, N, K, M)
+        ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+        assert L.mmhip_mul_mat_bias_add(t, ptr(W.data), N, K, W.row_bytes, ptr(x), K, M, ptr(bias), ptr(res), N, ptr(y),
+                                        N + pad, ptr(ws), need, stream()) == 0, L.mmhip_last_error()
+        assert rel_rms(y[:, :N], ref) < 4e-6
+        assert torch.isnan(y[:, N:]).all()
+    assert rel_rms(mm.mul_mat(W, x), prod) < 4e-6
+
+
+@pytest.mark.parametrize("t,N,K,M", [(Q8_0, 512, 2048, 40), (Q4_K, 4096, 2048, 100), (Q5_K, 768, 4096, 200),
+                                     (Q6_K, 2048, 2048, 64), (Q6_K, 6144, 768, 333), (Q8_0, 12288, 768, 1000)])
+def test_every_form_gives_the_same_sums(mm, pkg, t, N, K, M):
+    L = mm.load()
+    Ws = [weight(mm, pkg, t, N, K, 9200 + i) for i in range(2)]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9300 + M)
+    x = torch.randn((M, K), device="cuda", generator=g)
+    bias = torch.randn(N, device="cuda", generator=g)
+    xh = x.half()
+    plain = [mm.mul_mat(W, x) for W in Ws]
+    biased = mm.mul_mat_bias_add(Ws[0], x, bias)
+    assert torch.equal(biased, plain[0] + bias)
+    # f16 activations (with the workspace split K takes)
+    need = L.mmhip_mul_mat_h_workspace(t, N, K, M)
+    ws = torch.empty(max(need, 1), dtype=torch.uint8, device="cuda")
+    y = torch.empty((M, N), device="cuda")
+
+    def half_form():
+        assert L.mmhip_mul_mat_bias_add_hw(t, ptr(Ws[0].data), N, K, Ws[0].row_bytes, ptr(xh), M, None, None, 0, ptr(y), N,
+                                           ptr(ws) if need else None, need, stream()) == 0
+        return torch.equal(y, plain[0])
+
+    assert half_form()
+    # a registered f16 copy
+    copy = torch.empty(L.mmhip_weights_f16_bytes(N, K), dtype=torch.uint8, device="cuda")
+    assert L.mmhip_weights_to_f16(t, ptr(Ws[0].data), N, K, Ws[0].row_bytes, ptr(copy), stream()) == 0
+    assert torch.equal(copy.view(torch.float16).view(N, K), Ws[0].exact.half())
+    assert L.mmhip_register_weights_f16(ptr(Ws[0].data), N, K, ptr(copy)) == 0
+    try:
+        y.fill_(float("nan"))
+        assert half_form()
+    finally:
+        assert L.mmhip_unregister_weights_f16(ptr(Ws[0].data)) == 0
+    # two matrices in one launch
+    ys = [torch.empty((M, N), device="cuda") for _ in Ws]
+    arr = lambda c, v: (c * len(v))(*v)  # noqa: E731
+    assert L.mmhip_mul_mat_multi_h(t, 2, arr(ctypes.c_void_p, [W.data.data_ptr() for W in Ws]), N, K, Ws[0].row_bytes,
+                                   ptr(xh), M, None, arr(ctypes.c_void_p, [v.data_ptr() for v in ys]),
+                                   arr(ctypes.c_int64, [N, N]), stream()) == 0, L.mmhip_last_error()
+    if not need:  # split K is the plain form's only
+        assert all(torch.equal(a, b) for a, b in zip(ys, plain))
+        # the SwiGLU epilogue, either half first
+        for swapped in (False, True):
+            value, gate = (biased[:, N // 2:], biased[:, :N // 2]) if swapped else (biased[:, :N // 2], biased[:, N // 2:])
+            act = torch.empty((M, N // 2), device="cuda")
+            assert L.mmhip_swiglu(ctypes.byref(mm.view_of(gate)), ctypes.byref(mm.view_of(value)), 0, ptr(act),
+                                  stream()) == 0
+            h, hh = mm.mul_mat_bias_swiglu(Ws[0], x, bias, swapped, f32_out=True, f16_out=True)
+            assert torch.equal(h, act) and torch.equal(hh, act.half())
+
+
+@pytest.mark.parametrize("N,K,M,pad", [(300, 320, 70, 0), (6000, 768, 690, 8), (6144, 704, 1380, 0), (511, 512, 191, 16)])
+def test_bf16_tile_edges(mm, N, K, M, pad):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(9400 + M)
+    W = (torch.randn((N, K + pad), device="cuda", generator=g) * 0.02).bfloat16()
+    x = torch.randn((M, K), device="cuda", generator=g)
+    L = mm.load()
+    need = L.mmhip_mul_mat_workspace(30, N, K, M)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    y = torch.full((M, N + 5), float("nan"), device="cuda")
+    assert L.mmhip_mul_mat(30, ptr(W), N, K, 2 * (K + pad), ptr(x), K, M, ptr(y), N + 5, ptr(ws), need, stream()) == 0
+    assert rel_rms(y[:, :N], x.bfloat16().double() @ W[:, :K].double().T) < 4e-6
+    assert torch.isnan(y[:, N:]).all()
