@@ -187,6 +187,15 @@ int    mmhip_mul_mat_q(int type, const void * W, int64_t N, int64_t K, int64_t w
  * src/qwen3-lm.h:826-828, MLP down src/qwen3-lm.h:835-836); r may alias y. */
 int    mmhip_mul_mat_q_add(int type, const void * W, int64_t N, int64_t K, int64_t w_row_stride, const void * xq,
                            int64_t M, const float * r, int64_t ldr, float * y, int64_t ldy, void * stream);
+/* Several GEMVs of the same activation rows in one launch: n (2..3) Q8_0
+ * matrices of N rows x K, w_row_stride bytes apart, y[i][m*ldy[i] + r] =
+ * mul_mat_q of W[i], bit for bit (the depth decoder's q / k / v and gate / up
+ * projections, src/depth-decoder.h:206-208, :228-230).  M in 3..16, N a
+ * multiple of 16 up to 8192; mmhip_mul_mat_q_multi_supported says whether a
+ * shape is taken. */
+int    mmhip_mul_mat_q_multi_supported(int type, int n, int64_t N, int64_t K, int64_t w_row_stride, int64_t M);
+int    mmhip_mul_mat_q_multi(int type, int n, const void * const * W, int64_t N, int64_t K, int64_t w_row_stride,
+                             const void * xq, int64_t M, float * const * y, const int64_t * ldy, void * stream);
 /* The GEMV that follows an RMS norm, with the norm in its prologue: the
  * GGML_OP_RMS_NORM + GGML_OP_MUL by the norm weight of qwen3_rms_norm
  * (src/qwen3-lm.h:736, :834, :843) feeding the Q/K/V, gate/up and lm_head

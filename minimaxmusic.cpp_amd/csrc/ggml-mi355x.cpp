@@ -1020,7 +1020,7 @@ struct plan_step {
     int                  glu      = -1;  // MM: the SWIGLU node whose SwiGLU runs in the GEMV's prologue
     int                  glu_epi  = -1;  // MM / GEMM: the SWIGLU node computed in the GEMV's / GEMM's epilogue
     int                  glu_swapped = 0;  // GEMM: the gate rows are the first half
-    int                  multi[2]    = { -1, -1 };  // GEMM: further MUL_MATs of the same activations in this launch
+    int                  multi[2]    = { -1, -1 };  // GEMM / MM: further MUL_MATs of the same activations in this launch
     int                  mm       = -1;  // GEMM: the MUL_MAT node
     int                  bias     = -1;  // GEMM: the bias ADD node / LN: the ADD of the LayerNorm bias
     int                  bias_src = -1;  // index 0/1 of that ADD's vector operand
@@ -1546,7 +1546,7 @@ bool feeds_only(struct ggml_cgraph * g, const graph_info & gi, int e, int fa, in
 // chains' source rows or their outputs, its input rows not their outputs
 // (no fused ADD: the residual would be another operand to check).
 bool mm_commutes_with_head(struct ggml_cgraph * g, const plan_step & h, const plan_step & s) {
-    if (s.kind != ST_MM || s.add >= 0 || s.glu >= 0 || s.glu_epi >= 0) {
+    if (s.kind != ST_MM || s.add >= 0 || s.glu >= 0 || s.glu_epi >= 0 || s.multi[0] >= 0) {
         return false;
     }
     const struct ggml_tensor * mm = ggml_graph_node(g, s.node);
@@ -1941,6 +1941,30 @@ graph_plan build_plan(struct ggml_cgraph * g) {
                 }
             }
         }
+        // A MUL_MAT o (node j) may join an earlier one's launch, its output
+        // written early: its memory must hold no other tensor of the graph (a
+        // buffer the allocator shares with anything else, live before o or
+        // not, keeps the launches separate), and no node between the two may
+        // write its operands.
+        auto written_early = [&](int j, const struct ggml_tensor * w) {
+            const struct ggml_tensor * o = ggml_graph_node(g, j);
+            auto own   = [&](const struct ggml_tensor * v) { return v == o || v->view_src == o; };
+            bool clear = !overlaps(o, w) && !overlaps(o, o->src[0]);
+            for (int t = i + 1; t < j && clear; t++) {
+                const struct ggml_tensor * u = ggml_graph_node(g, t);
+                const bool view = u->op == GGML_OP_VIEW || u->op == GGML_OP_RESHAPE || u->op == GGML_OP_PERMUTE ||
+                                  u->op == GGML_OP_TRANSPOSE || u->op == GGML_OP_NONE;
+                clear           = view || (!overlaps(u, o->src[0]) && !overlaps(u, o->src[1]));
+            }
+            for (int t = 0; t < gi.nn && clear; t++) {
+                const struct ggml_tensor * u = ggml_graph_node(g, t);
+                clear = own(u) || !overlaps(o, u);
+                for (int q = 0; q < GGML_MAX_SRC && clear; q++) {
+                    clear = !u->src[q] || own(u->src[q]) || !overlaps(o, u->src[q]);
+                }
+            }
+            return clear;
+        };
         // GEMM with the bias ADD and / or residual ADD that follow it in its store
         if (n->op == GGML_OP_MUL_MAT && !mm_is_gemv(n) && supports_mul_mat(n) && ggml_is_contiguous(n)) {
             plan_step st;
@@ -1992,19 +2016,7 @@ graph_plan build_plan(struct ggml_cgraph * g) {
                         !ggml_is_contiguous(o) || !ggml_are_same_shape(o, n) || n->src[0]->ne[1] % 256 != 0) {
                         continue;
                     }
-                    // o is written early: its memory must hold no other tensor of
-                    // the graph (a buffer the allocator shares with anything else,
-                    // live before j or not, keeps the launches separate)
-                    auto own = [&](const struct ggml_tensor * v) { return v == o || v->view_src == o; };
-                    bool clear = !overlaps(o, n->src[0]) && !overlaps(o, o->src[0]);
-                    for (int t = 0; t < gi.nn && clear; t++) {
-                        const struct ggml_tensor * u = ggml_graph_node(g, t);
-                        clear = own(u) || !overlaps(o, u);
-                        for (int q = 0; q < GGML_MAX_SRC && clear; q++) {
-                            clear = !u->src[q] || own(u->src[q]) || !overlaps(o, u->src[q]);
-                        }
-                    }
-                    if (!clear) {
+                    if (!written_early(j, n->src[0])) {
                         continue;
                     }
                     st.multi[nm++] = j;
@@ -2103,6 +2115,31 @@ graph_plan build_plan(struct ggml_cgraph * g) {
             // (a BF16 GEMV without a fusion too: the persistent decode kernel
             // streams the rows faster than the node's plain BF16 GEMV, e.g.
             // the lm_head behind the final norm, whose rows are a graph output)
+            if (st.slot_in >= 0 && st.add < 0 && st.norm < 0 && st.glu < 0 && st.src == -1) {
+                // further GEMVs on the same quantised rows with the same weight
+                // shape join this launch
+                const struct ggml_tensor * w  = n->src[0];
+                const int64_t              M  = n->src[1]->ne[1] * n->src[1]->ne[2] * n->src[1]->ne[3];
+                int                        nm = 0;
+                for (int j = i + 1; j < gi.nn && nm < 2; j++) {
+                    const struct ggml_tensor * o = ggml_graph_node(g, j);
+                    if (o->op != GGML_OP_MUL_MAT || o->src[1] != n->src[1] || absorbed[(size_t) j] ||
+                        o->src[0]->type != w->type || o->src[0]->ne[0] != w->ne[0] || o->src[0]->ne[1] != w->ne[1] ||
+                        o->src[0]->nb[1] != w->nb[1] || w->ne[2] != 1 || w->ne[3] != 1 || o->src[0]->ne[2] != 1 ||
+                        o->src[0]->ne[3] != 1 || !ggml_is_contiguous(n) || !ggml_is_contiguous(o) || !mm_is_gemv(o) ||
+                        !supports_mul_mat(o) || ((uintptr_t) w->data) % 16 != 0 ||
+                        ((uintptr_t) o->src[0]->data) % 16 != 0 ||
+                        (gi.uses[(size_t) j] == 1 && ggml_graph_node(g, gi.cons[(size_t) j])->op == GGML_OP_ADD) ||
+                        !mmhip_mul_mat_q_multi_supported(w->type, 2, w->ne[1], w->ne[0], (int64_t) w->nb[1], M) ||
+                        getenv("GGML_MI355X_DISABLE_GEMV_MULTI") || !written_early(j, w)) {
+                        continue;
+                    }
+                    st.multi[nm++] = j;
+                }
+                for (int k = 0; k < nm; k++) {
+                    absorbed[(size_t) st.multi[k]] = 1;
+                }
+            }
             if (st.slot_in >= 0 || st.add >= 0 || st.norm >= 0 || st.glu >= 0 || mm_is_bf16_dec(n)) {
                 absorbed[(size_t) i] = 1;
                 add_pending(st);
@@ -2457,6 +2494,19 @@ int run_step(mi_backend * c, struct ggml_cgraph * g, const plan_step & st, char 
                 if (rc != MMHIP_OK) {
                     break;
                 }
+            }
+            if (st.multi[0] >= 0) {
+                const void * wm[3] = { w->data, nullptr, nullptr };
+                float *      ym[3] = { (float *) n->data, nullptr, nullptr };
+                int64_t      lm[3] = { N, N, N };
+                int          nmat  = 1;
+                for (int k = 0; k < 2 && st.multi[k] >= 0; k++, nmat++) {
+                    const struct ggml_tensor * o = ggml_graph_node(g, st.multi[k]);
+                    wm[nmat] = o->src[0]->data;
+                    ym[nmat] = (float *) o->data;
+                }
+                rc = mmhip_mul_mat_q_multi(w->type, nmat, wm, N, K, (int64_t) w->nb[1], slot + st.slot_in, M, ym, lm, s);
+                break;
             }
             if (st.add >= 0) {
                 const struct ggml_tensor * r = ggml_graph_node(g, st.add)->src[st.add_res];

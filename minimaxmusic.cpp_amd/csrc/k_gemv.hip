@@ -127,12 +127,24 @@ template <bool AL> __device__ __forceinline__ uint2 ld8a(const uint8_t * p) {
 // the decode shapes: this beats both a per-chunk loop and a split of K over
 // the workgroup's waves, which adds a barrier and an LDS reduction).  The
 // activation chunks come through L1/L2 (a few KB shared by every wave).
-template <int NC, int R, int CH, bool ONE>  // ONE: K <= 1024 * CH, a single pass
+template <int NC, int R, int CH, bool ONE, bool MULTI = false>  // ONE: K <= 1024 * CH, a single pass
 __global__ __launch_bounds__(256) void k_gemv_q8_0(const uint8_t * __restrict__ W, int64_t N, int64_t K, int64_t rs,
                                                     const int8_t * __restrict__ xq, const float * __restrict__ xd,
-                                                    float * y, int64_t ldy, const float * res, int64_t ldr) {
-    const int     lane = threadIdx.x & 63;
-    const int64_t g    = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
+                                                    float * y, int64_t ldy, const float * res, int64_t ldr,
+                                                    const QMulti m) {
+    const int lane = threadIdx.x & 63;
+    int64_t   g    = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
+    if constexpr (MULTI) {  // R = 1: wave g takes row g of the m.n matrices' rows laid end to end
+        const int gw = __builtin_amdgcn_readfirstlane((int) g);
+        const int i  = gw >= 2 * (int) N ? 2 : gw >= (int) N ? 1 : 0;
+        if (gw >= m.n * (int) N) {
+            return;
+        }
+        g   = gw - i * (int) N;
+        W   = i == 0 ? m.W[0] : i == 1 ? m.W[1] : m.W[2];
+        y   = i == 0 ? m.y[0] : i == 1 ? m.y[1] : m.y[2];
+        ldy = i == 0 ? m.ldy[0] : i == 1 ? m.ldy[1] : m.ldy[2];
+    }
     if (g * R >= N) {
         return;
     }
@@ -1145,15 +1157,44 @@ struct MfArgs {
     int64_t         ldy;
     const float *   res;
     int64_t         ldr;
+    // up to two more matrices of the same shape (N a multiple of 16): row
+    // groups [i gper, (i + 1) gper) are matrix i's
+    int64_t         gper;  // 0: the one matrix
+    const uint8_t * W1, * W2;
+    float *         y1, * y2;
+    int64_t         ldy1, ldy2;
 };
+
+// the matrix of row group g (g becomes the group inside it)
+__device__ __forceinline__ const uint8_t * mf_matrix(const MfArgs & a, int64_t & g, float *& y, int64_t & ldy) {
+    const uint8_t * W = a.W;
+    y                 = a.y;
+    ldy               = a.ldy;
+    if (a.gper > 0 && g >= a.gper) {
+        g -= a.gper;
+        W   = a.W1;
+        y   = a.y1;
+        ldy = a.ldy1;
+        if (g >= a.gper) {
+            g -= a.gper;
+            W   = a.W2;
+            y   = a.y2;
+            ldy = a.ldy2;
+        }
+    }
+    return W;
+}
 
 // chunk starting at pair p0 of row group g: weight pieces and row scales
 // (rows past N re-read row N - 1; chunks past the wave's range are not
 // loaded, their buffers not used)
 __device__ __forceinline__ void mf_load(MfChunk & b, const MfArgs & a, int64_t g, int p0, int r, int q) {
-    const int64_t row0 = g * 16;
+    float *         y;
+    int64_t         ldy;
+    const uint8_t * W    = mf_matrix(a, g, y, ldy);
+    const int64_t   row0 = g * 16;
     const __amdgpu_buffer_rsrc_t rr = __builtin_amdgcn_make_buffer_rsrc(
-        (void *) (a.W + row0 * a.rs), (short) 0, (int) (min((int64_t) 16, a.N - row0) * a.rs), 0x00020000);
+        (void *) (W + row0 * a.rs), (short) 0, (int) (min((int64_t) 16, a.N - row0) * a.rs), 0x00020000);
     const int      nr = (int) min((int64_t) 16, a.N - row0);
     const unsigned wo = (unsigned) (min(r, nr - 1) * (int) a.rs + 16 * q);
 #pragma unroll
@@ -1225,7 +1266,7 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q8_0_mfma(MfArgs a) {
     const int nch   = (np + MF_PC - 1) / MF_PC;                  // chunks per row, split over the waves
     const int cb    = wv * nch / PG_WAVES, ce = (wv + 1) * nch / PG_WAVES;
     const int pe    = min(ce * MF_PC, np);  // the wave's pairs: [cb MF_PC, pe)
-    const int64_t ng = (a.N + 15) / 16;
+    const int64_t ng = a.gper > 0 ? a.gper * (a.W2 ? 3 : 2) : (a.N + 15) / 16;
     // 1. the M columns and their block scales DMA'd into LDS (global_load_lds,
     // issued first: they return first), 1 KB of a column or 64 scales per
     // instruction, instructions dealt round-robin to the waves; columns past
@@ -1274,7 +1315,10 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q8_0_mfma(MfArgs a) {
         // order: loaded after the next group's rows it would wait for them)
         const int     ocol = (int) (threadIdx.x >> 4) & 15, orr = threadIdx.x & 15;
         const int     ol = orr + 16 * (ocol >> 2), oi = ocol & 3;
-        const int64_t orow = gc * 16 + orr;
+        int64_t       gy = gc, ldy;
+        float *       y;
+        (void) mf_matrix(a, gy, y, ldy);
+        const int64_t orow = gy * 16 + orr;
         const bool    ost  = threadIdx.x < 256 && ocol < a.M && orow < a.N;
         const float   ores = ost && a.res ? a.res[ocol * a.ldr + orow] : 0.0f;
 #pragma unroll
@@ -1299,7 +1343,7 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q8_0_mfma(MfArgs a) {
                 t += s_pt[(w * 4 + oi) * 64 + ol];
             }
             if (ost) {
-                a.y[ocol * a.ldy + orow] = a.res ? t + ores : t;
+                y[ocol * ldy + orow] = a.res ? t + ores : t;
             }
         }
         lds_barrier();  // the partial sums are read before the next group writes them
@@ -1323,7 +1367,7 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q8_0_mfma(MfArgs a) {
 static int64_t pg_cus();
 
 template <int MAXC> static int launch_mf(const MfArgs & a, hipStream_t stream) {
-    const int64_t ng   = (a.N + 15) / 16;
+    const int64_t ng   = a.gper > 0 ? a.gper * (a.W2 ? 3 : 2) : (a.N + 15) / 16;
     const int64_t wgs  = std::min<int64_t>(ng, pg_cus());
     const size_t  lds  = (size_t) 16 * (a.K + MF_PAD) + (size_t) 16 * (a.K / 32) * 4 + (size_t) PG_WAVES * 4 * 64 * 4;
     auto          kern = k_gemv_q8_0_mfma<MAXC>;
@@ -1699,10 +1743,10 @@ static int launch_q8_0(const uint8_t * W, int64_t N, int64_t K, int64_t rs, cons
                        const float * r, int64_t ldr, hipStream_t stream) {
     if (K <= 1024 * CH) {
         auto kern = k_gemv_q8_0<NC, R, CH, true>;
-        return launch_gemv(kern, R, N, stream, W, N, K, rs, x.qs, x.d, y, ldy, r, ldr);
+        return launch_gemv(kern, R, N, stream, W, N, K, rs, x.qs, x.d, y, ldy, r, ldr, QMulti{});
     }
     auto kern = k_gemv_q8_0<NC, R, CH, false>;
-    return launch_gemv(kern, R, N, stream, W, N, K, rs, x.qs, x.d, y, ldy, r, ldr);
+    return launch_gemv(kern, R, N, stream, W, N, K, rs, x.qs, x.d, y, ldy, r, ldr, QMulti{});
 }
 
 template <int NC, int R>
@@ -1842,6 +1886,57 @@ static bool gemv_q6_pro_ok(int64_t K, int64_t M, int64_t rs, const void * W);
 static int  gemv_q6_pro(const void * W, int64_t N, int64_t K, int64_t rs, const ActPtrs & x, int64_t M, float * y,
                         int64_t ldy, hipStream_t stream, const float * r, int64_t ldr);
 
+// The shapes the int8-MFMA GEMV takes.
+static bool gemv_mf_ok(int64_t K, int64_t M, int64_t rs) {
+    static const bool mfma = getenv("GGML_MI355X_DISABLE_GEMV_MFMA") == nullptr;
+    return mfma && (M >= 9 || (M >= 3 && K > 4096)) && M <= 16 && K % 1024 == 0 && K <= 16 * 3 * MF_PC * 64 &&
+           rs % 16 == 0;
+}
+
+// Up to three Q8_0 matrices of one shape against the same 3..16 activation
+// columns in one launch (the depth decoder's q / k / v and its gate / up,
+// src/depth-decoder.h:206-230): a launch and the activations' staging are paid
+// once, and the rows of all of them fill the CUs (three 4096 x 4096 on 16
+// columns: one group of 16 rows per CU and launch).  The sums are the separate
+// calls', to the bit.  Depth layer, two sequences of 8 rows: 431 -> 357 us per
+// four layers against a launch per matrix.
+bool gemv_q8_multi_ok(int n, int64_t N, int64_t K, int64_t M, int64_t rs) {
+    return n >= 2 && n <= 3 && M >= 3 && M <= 16 && N % 16 == 0 && N > 0 && N <= 8192 && K % 256 == 0 && K > 0 &&
+           rs % 16 == 0 && rs >= row_bytes(TYPE_Q8_0, K) && (gemv_mf_ok(K, M, rs) || (M <= 8 && K <= 4096));
+}
+
+template <int NC>
+static int launch_q8_0_multi(const QMulti & m, int64_t N, int64_t K, int64_t rs, const ActPtrs & x, hipStream_t stream) {
+    constexpr int CH = NC > 4 ? 2 : 4;
+    if (K <= 1024 * CH) {
+        return launch_gemv(k_gemv_q8_0<NC, 1, CH, true, true>, 1, m.n * N, stream, nullptr, N, K, rs, x.qs, x.d, nullptr, 0,
+                           nullptr, 0, m);
+    }
+    return launch_gemv(k_gemv_q8_0<NC, 1, CH, false, true>, 1, m.n * N, stream, nullptr, N, K, rs, x.qs, x.d, nullptr, 0,
+                           nullptr, 0, m);
+}
+
+int gemv_q8_multi(const QMulti & m, int64_t N, int64_t K, int64_t rs, const ActPtrs & x, int64_t M, hipStream_t stream) {
+    if (!gemv_q8_multi_ok(m.n, N, K, M, rs) || (uintptr_t) x.qs % 16 != 0 || (uintptr_t) x.d % 16 != 0) {
+        return set_error(MMHIP_ERR_UNSUPPORTED, "gemv (several matrices): n=%d N=%lld K=%lld M=%lld not supported", m.n,
+                         (long long) N, (long long) K, (long long) M);
+    }
+    if (gemv_mf_ok(K, M, rs)) {
+        const bool   three = m.n > 2;
+        const MfArgs a{ m.W[0], N, (int) K, rs, x.qs, x.d, (int) M, m.y[0], m.ldy[0], nullptr, 0, N / 16, m.W[1],
+                        three ? m.W[2] : nullptr, m.y[1], three ? m.y[2] : nullptr, m.ldy[1], three ? m.ldy[2] : 0 };
+        return K <= 16 * 2 * MF_PC * 64 ? launch_mf<2>(a, stream) : launch_mf<3>(a, stream);
+    }
+    switch (M) {
+        case 3: return launch_q8_0_multi<3>(m, N, K, rs, x, stream);
+        case 4: return launch_q8_0_multi<4>(m, N, K, rs, x, stream);
+        case 5: return launch_q8_0_multi<5>(m, N, K, rs, x, stream);
+        case 6: return launch_q8_0_multi<6>(m, N, K, rs, x, stream);
+        case 7: return launch_q8_0_multi<7>(m, N, K, rs, x, stream);
+        default: return launch_q8_0_multi<8>(m, N, K, rs, x, stream);
+    }
+}
+
 int gemv_q(int wtype, const void * W, int64_t N, int64_t K, int64_t rs, const ActPtrs & x, int64_t M, float * y,
            int64_t ldy, hipStream_t stream, const float * r, int64_t ldr) {
     if (!gemv_supported(wtype, N, K, rs, W) || M < 1 || ldy < N) {
@@ -1859,12 +1954,9 @@ int gemv_q(int wtype, const void * W, int64_t N, int64_t K, int64_t rs, const Ac
     // the int8-MFMA GEMV at 9..16 columns, and at 3..8 columns for rows longer
     // than 4096 (shorter rows at <= 8 columns: the column-group GEMV below is
     // faster, one row per wave with no LDS staging or cross-wave sum)
-    static const bool mfma = getenv("GGML_MI355X_DISABLE_GEMV_MFMA") == nullptr;
-    if (mfma && wtype == TYPE_Q8_0 && (M >= 9 || (M >= 3 && K > 4096)) && M <= 16 && K % 1024 == 0 &&
-        K <= 16 * 3 * MF_PC * 64 &&
-        rs % 16 == 0 &&
-        (uintptr_t) W % 16 == 0 && (uintptr_t) x.qs % 16 == 0 && (uintptr_t) x.d % 16 == 0) {
-        const MfArgs a{ wb, N, (int) K, rs, x.qs, x.d, (int) M, y, ldy, r, ldr };
+    if (wtype == TYPE_Q8_0 && gemv_mf_ok(K, M, rs) && (uintptr_t) W % 16 == 0 && (uintptr_t) x.qs % 16 == 0 &&
+        (uintptr_t) x.d % 16 == 0) {
+        const MfArgs a{ wb, N, (int) K, rs, x.qs, x.d, (int) M, y, ldy, r, ldr, 0, nullptr, nullptr, nullptr, nullptr, 0, 0 };
         return K <= 16 * 2 * MF_PC * 64 ? launch_mf<2>(a, stream) : launch_mf<3>(a, stream);
     }
     if (wtype == TYPE_Q8_0 && M > 8 && M <= 16 && K <= 8192 && K % 32 == 0) {
@@ -2185,6 +2277,32 @@ extern "C" int mmhip_mul_mat_bf16_dec(const void * W, int64_t N, int64_t K, int6
     const int epi = glu ? 2 : r ? 1 : 0;
     return M == 1 ? bf16_dec_dispatch<1>(a, norm_w != nullptr, epi, (hipStream_t) stream)
                   : bf16_dec_dispatch<2>(a, norm_w != nullptr, epi, (hipStream_t) stream);
+}
+
+extern "C" int mmhip_mul_mat_q_multi_supported(int type, int n, int64_t N, int64_t K, int64_t w_row_stride, int64_t M) {
+    return type == TYPE_Q8_0 && gemv_q8_multi_ok(n, N, K, M, w_row_stride) ? 1 : 0;
+}
+
+extern "C" int mmhip_mul_mat_q_multi(int type, int n, const void * const * W, int64_t N, int64_t K, int64_t w_row_stride,
+                                     const void * xq, int64_t M, float * const * y, const int64_t * ldy,
+                                     void * stream) {
+    MMHIP_API_BEGIN();
+    if (!W || !xq || !y || !ldy || !mmhip_mul_mat_q_multi_supported(type, n, N, K, w_row_stride, M)) {
+        return set_error(MMHIP_ERR_UNSUPPORTED, "mul_mat_q_multi: type %d n=%d N=%lld K=%lld M=%lld", type, n,
+                         (long long) N, (long long) K, (long long) M);
+    }
+    QMulti m;
+    m.n = n;
+    for (int i = 0; i < n; i++) {
+        if (!W[i] || !y[i] || ldy[i] < N || ((uintptr_t) W[i]) % 16 != 0) {
+            return set_error(MMHIP_ERR_INVALID, "mul_mat_q_multi: matrix %d: null or unaligned operand", i);
+        }
+        m.W[i]   = (const uint8_t *) W[i];
+        m.y[i]   = y[i];
+        m.ldy[i] = ldy[i];
+    }
+    const ActLayout L = act_layout(type, K, M);
+    return gemv_q8_multi(m, N, K, w_row_stride, ActPtrs::from(L, xq), M, (hipStream_t) stream);
 }
 
 extern "C" int mmhip_mul_mat_q(int type, const void * W, int64_t N, int64_t K, int64_t w_row_stride, const void * xq,

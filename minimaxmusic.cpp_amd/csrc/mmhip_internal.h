@@ -78,6 +78,17 @@ bool gemv_supported(int wtype, int64_t N, int64_t K, int64_t row_stride, const v
 int  gemv_q(int wtype, const void * W, int64_t N, int64_t K, int64_t row_stride, const ActPtrs & x, int64_t M, float * y,
             int64_t ldy, hipStream_t stream, const float * r = nullptr, int64_t ldr = 0);
 
+// Up to three Q8_0 matrices of N rows against the same 3..16 quantised
+// columns in one launch.
+struct QMulti {
+    int             n = 0;
+    const uint8_t * W[3]{};
+    float *         y[3]{};
+    int64_t         ldy[3]{};
+};
+bool gemv_q8_multi_ok(int n, int64_t N, int64_t K, int64_t M, int64_t rs);
+int  gemv_q8_multi(const QMulti & m, int64_t N, int64_t K, int64_t rs, const ActPtrs & x, int64_t M, hipStream_t stream);
+
 // MFMA GEMM with in-LDS dequantisation (any M); the workspace holds the f16
 // copy of the activations (gemm_workspace bytes, 16-byte aligned).
 size_t gemm_workspace(int64_t K, int64_t M);

@@ -1,0 +1,86 @@
+"""GPU: several Q8_0 GEMVs of the same activation rows in one launch
+(mmhip_mul_mat_q_multi, the depth decoder's q / k / v and gate / up,
+src/depth-decoder.h:206-230), bit for bit the separate calls: 3..8 columns on
+the one-row-per-wave kernel, 9..16 (and 3..8 on long rows) on the int8 MFMA;
+and a depth layer whose graph joins them, bit for bit the one that does not."""
+import ctypes
+import importlib
+import os
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def ptr(t):
+    return ctypes.c_void_p(t.data_ptr())
+
+
+def arr(ctype, vals):
+    return (ctype * len(vals))(*vals)
+
+
+@pytest.mark.parametrize("n,N,K,M", [(3, 4096, 4096, 16), (2, 6144, 4096, 9), (3, 16, 1024, 12), (2, 4112, 6144, 5),
+                                     (3, 4096, 4096, 8), (2, 6144, 4096, 3), (3, 48, 256, 4), (2, 8192, 2304, 7)])
+def test_multi_equals_separate(mm, pkg, n, N, K, M):
+    L = mm.load()
+    Ws = [mm.QuantWeight.from_gguf(mm.Q8_0, pkg.synth.gguf_blocks_np(mm.Q8_0, N, K, 40 + i), N, K) for i in range(n)]
+    x = torch.from_numpy(pkg.synth.normal_np((M, K), 50 + M)).cuda()
+    xq = mm.quantize_act(mm.Q8_0, x)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert L.mmhip_mul_mat_q_multi_supported(mm.Q8_0, n, N, K, Ws[0].row_bytes, M) == 1
+    refs = [mm.mul_mat(W, x) for W in Ws]
+    ys = [torch.full((M, N + 4 * i), float("nan"), device="cuda") for i in range(n)]
+    assert L.mmhip_mul_mat_q_multi(mm.Q8_0, n, arr(ctypes.c_void_p, [W.data.data_ptr() for W in Ws]), N, K,
+                                   Ws[0].row_bytes, ptr(xq), M, arr(ctypes.c_void_p, [y.data_ptr() for y in ys]),
+                                   arr(ctypes.c_int64, [y.shape[1] for y in ys]), st) == 0, L.mmhip_last_error()
+    for y, r in zip(ys, refs):
+        assert torch.equal(y[:, :N], r)
+        assert torch.isnan(y[:, N:]).all()
+
+
+def test_multi_rejects(mm):
+    L = mm.load()
+    P = arr(ctypes.c_void_p, [16, 16, 16])
+    ld = arr(ctypes.c_int64, [4096] * 3)
+    p = ctypes.c_void_p(16)
+    for type_, n, N, K, M in [(12, 2, 4096, 4096, 16), (8, 1, 4096, 4096, 16), (8, 4, 4096, 4096, 16),
+                              (8, 2, 4100, 4096, 16), (8, 2, 4096, 4096, 17), (8, 2, 4096, 4096, 2),
+                              (8, 2, 8208, 4096, 16)]:
+        assert L.mmhip_mul_mat_q_multi(type_, n, P, N, K, K // 32 * 34, p, M, P, ld, None) != 0
+
+
+@pytest.mark.parametrize("S,B", [(8, 2), (3, 1), (2, 2)])
+def test_depth_layer_with_and_without(pkg, S, B):
+    og = importlib.import_module(pkg.__name__ + ".opgraph")
+    dg = importlib.import_module(pkg.__name__ + ".depthgraph")
+    w = dg.synth_layer(77)
+    x = np.random.default_rng(78).standard_normal((B, S, dg.DIM)).astype(np.float32)
+
+    def run():
+        g = og.OpGraph(n_tensors=128)
+        try:
+            lw = dg.Layer(g)
+            tx = g.tensor(og.F32, [dg.DIM, S, B])
+            out = dg.build_layer(g, lw, tx, S, B)
+            g.build([out])
+            lw.upload(g, w)
+            g.set(tx, x)
+            ys = []
+            for _ in range(3):  # eager, captured, replayed
+                g.compute()
+                ys.append(g.get(out))
+            assert all(np.array_equal(y, ys[0]) for y in ys)
+            return ys[0]
+        finally:
+            g.close()
+
+    joined = run()
+    os.environ["GGML_MI355X_DISABLE_GEMV_MULTI"] = "1"
+    try:
+        separate = run()
+    finally:
+        del os.environ["GGML_MI355X_DISABLE_GEMV_MULTI"]
+    assert np.isfinite(joined).all() and np.array_equal(joined, separate)
