@@ -20,8 +20,10 @@
 // masked KV tiles (the causal upper triangle, the -inf padding of the cache
 // window) are never read.
 //
-// The unmasked D = 128 case on a full grid (the DiT) runs k_fa_dma instead,
-// described above its definition below.
+// Unmasked attention (the DiT) and the masked D = 128 case on a full grid run
+// k_fa_dma instead, described above its definition below; this kernel keeps
+// the masked calls on smaller grids or at D = 64, and rows that are not
+// 16-byte aligned.
 #include <type_traits>
 
 #include "k_fa_common.h"
@@ -338,15 +340,14 @@ __global__ __launch_bounds__(NW * 64) void k_fa_mfma(FaArgs a, const int * __res
 }
 
 // ---------------------------------------------------------------------------
-// Unmasked D = 128 with a full grid (the DiT's attention, src/dit.h:221-222):
-// k_fa_dma.  The chip runs MFMA work at a power-limited clock that drops
+// Unmasked attention (the DiT's, src/dit.h:221-222): k_fa_dma.  The chip runs MFMA work at a power-limited clock that drops
 // further with every VALU op and LDS byte issued beside it, so this kernel
 // minimises both per MFMA:
-//  - K / V tiles (64 keys, 16 KB each) go from global memory straight into a
-//    double-buffered LDS ring with global_load_lds (no register staging, no
-//    transposing stores); K rows store 16-byte chunk c at c ^ (row & 15), V
-//    rows at c ^ 2 (row & 3), which keeps both read patterns bank-conflict
-//    free;
+//  - K / V tiles (64 keys, 16 KB each at D = 128) go from global memory
+//    straight into an LDS ring with global_load_lds (no register staging, no
+//    transposing stores); K rows store 16-byte chunk c at c ^ (row & 15)
+//    (D = 64: c ^ (row / 2 & 7)), V rows at c ^ 2 (row & 3), which keeps both
+//    read patterns bank-conflict free;
 //  - V^T operands come from ds_read_b64_tr_b16: within each 16-lane group,
 //    lane i receives element i % 4 of the 4-element rows addressed by lanes
 //    4 j + i / 4 (j = 0..3), so the lanes address V rows in exactly the key
@@ -355,20 +356,34 @@ __global__ __launch_bounds__(NW * 64) void k_fa_mfma(FaArgs a, const int * __res
 //    accumulator starts at -m (the running row max, log2 units): the scores
 //    come out as s - m and p = exp2(s - m) is one v_exp per score; the row
 //    sum adds the f16 p pairs with v_dot2 (the same values the PV MFMA uses);
-//  - the running max moves only on a slow path: on a row's first 32 keys, or
+//  - the running max moves only on a slow path: on a row's first unit, or
 //    when a lane's partial sum exceeds 2^14 (some score more than 14 above
 //    m); O and l are then rescaled by exp2(-shift).  p stays below 2^15,
 //    inside f16.
-// Pipeline per wave (32 query rows, 8 waves, two per SIMD): unit u = 32 keys;
-// unit u runs the softmax of unit u (VALU) between the MFMAs of QK(u + 1) and
-// PV(u - 1), with the LDS operands of MFMA step i + 2 read during step i.  One
-// barrier per 64-key tile.
+// Pipeline per wave (32 query rows): a unit is 32 keys (UK = 1, D = 128) or 64
+// (UK = 2, D = 64: two score chains, so that the 8 + 8 short MFMA steps cover
+// each other's latency); unit u runs the softmax of unit u (VALU) between the
+// MFMAs of QK(u + 1) and PV(u - 1), with the LDS operands of MFMA step i + PF
+// read during step i.  Two units alternate between two sets of score and P
+// registers (copying them cost 56 VALU moves per 32 keys).  One barrier per
+// 64-key tile.
+//
+// Workgroups of 8 waves (256 query rows) when those give every CU one, else
+// of 4 waves (128 rows).  Measured, register-staged kernel -> this one:
+// D = 64, Hq = 32, B = 2: S = 690 25.1 -> 18.8 us, S = 4000 423 -> 303 us,
+// S = 250 (B = 1) 9.8 -> 7.6 us; D = 128, Hq = 16: S = 690 (B = 2) 28.0 ->
+// 21.8 us, S = 1500 (B = 1) 51.2 -> 37.3 us; S = 60 (B = 1) 6.9 -> 6.0 us.
+// S = 4096, D = 128, B = 2: 273 us (1.0 PFLOP/s).  At S = 690 (1.4 waves a
+// SIMD) a wave's own chain of LDS reads, MFMAs and exponentials is what takes
+// the time, at S = 4000 the MFMA and exponential issue.
 __device__ __forceinline__ void fa_dma16(const void * src, uint32_t lds_addr) {
     // issued from inline asm: the compiler's wait-count tracking would
     // otherwise wait for the DMA before unrelated LDS reads; the kernel waits
     // for it itself before the barrier that publishes a tile
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(lds_addr) : "memory", "m0");
 }
+
+__device__ const uint4 fa_zeros[1] = {};
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) short4_t lds_short4_t;
@@ -382,21 +397,25 @@ typedef __attribute__((address_space(3))) short4_t lds_short4_t;
 // units) to its scores, loaded while the unit before it runs.  A row's
 // running max is set on its first unit with a visible key.
 //
-// The unmasked form stages K and V through 4-tile rings (128 KB of LDS, one
-// workgroup per CU as the registers allow anyway), each tile issued three
+// The unmasked form stages K and V through 4-tile rings (128 KB of LDS at
+// D = 128, 64 KB at D = 64), each tile issued three
 // 64-key steps before its first reader and waited for by count, so the
 // loads of the two younger steps stay in flight across a barrier.  The
 // masked form's rings hold 2 tiles (64 KB, two workgroups per CU): the K
 // tile of the next step and the V tile of this one are waited for at each
 // step's barrier.
-template <bool MASK, int NW = 8, int KR = 4>
+template <bool MASK, int D, int NW, int KR, int UK>
 __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __restrict__ row_end,
                                                        const int * __restrict__ zero_end, int n_qtiles,
                                                        float * __restrict__ out) {
-    constexpr int D = 128, NQK = 8, NDB = 4, TILE = FA_BK * 256;
-    constexpr int US  = 1;         // unit stride of a wave
-    constexpr int PPW = 16 / NW;   // 1 KB pieces of a 16 KB tile each wave DMAs
-    static_assert(MASK ? (NW == 4 && KR == 2) : (NW == 8 && KR == 4), "configurations");
+    constexpr int NQK = D / 16, NDB = D / 32;  // 16-dim steps of QK; 32-dim blocks of O
+    constexpr int RB = 2 * D, TILE = FA_BK * RB;  // bytes of a row and of a tile
+    constexpr int RCH = RB / 16, RPP = 1024 / RB; // 16-byte chunks of a row, rows of a 1 KB piece
+    constexpr int US = 1, UB = 32 * UK;           // unit stride of a wave, keys of a unit
+    constexpr int NS = NQK * UK;                  // MFMA steps of QK (and of PV) per unit
+    constexpr int PPW = TILE / 1024 / NW;         // 1 KB pieces of a tile each wave DMAs
+    static_assert((D == 64 || D == 128) && PPW >= 1 && (MASK ? KR == 2 : KR == 4) &&
+                  (UK == 1 || (UK == 2 && D == 64 && !MASK)), "configurations");
     extern __shared__ __attribute__((aligned(1024))) char smem[];  // K ring, then V ring
     const int  total = n_qtiles * a.Hq * a.B;
     // one 128-row tile per workgroup (masked, four waves): workgroups in
@@ -415,12 +434,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
     const int  lq    = lane & 31;
     const int  hh    = lane >> 5;
     const int   par  = 0;  // the wave's first unit
-    int         my_q;
-    if constexpr (MASK) {
-        my_q = qt * 128 + wave * 32 + lq;
-    } else {
-        my_q = qt * 256 + wave * 32 + lq;
-    }
+    const int   my_q = qt * (32 * NW) + wave * 32 + lq;
     const bool  q_ok = my_q < a.nq;
     const float log2e = 1.4426950408889634f;
     const float sl2   = a.scale * log2e;
@@ -478,8 +492,8 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
     float l = 0.0f;  // this lane's half of the row sum
     bool  mset = false;                           // (MASK) the running max is set for this lane's row
     const int n     = (kv_end + FA_BK - 1) / FA_BK;  // 64-key tiles staged
-    const int nu_wg = (kv_end + 31) / 32;            // 32-key units staged
-    const int nu    = (w_end + 31) / 32;             // 32-key units the wave's rows see
+    const int nu_wg = (kv_end + UB - 1) / UB;        // units staged
+    const int nu    = (w_end + UB - 1) / UB;         // units the wave's rows see
     const int nk    = nu;                            // units this wave computes
 
     // the mask of this lane's query at the 16 keys of unit u it holds
@@ -513,36 +527,40 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
         }
     };
 
-    // DMA: this wave fills 1 KB pieces PPW wave .. PPW wave + PPW - 1 (4 rows
-    // each) of a K and a V tile; lane -> row 4 piece + lane / 16, stored chunk
-    // lane % 16
+    // DMA: this wave fills 1 KB pieces PPW wave .. PPW wave + PPW - 1 (RPP rows
+    // each) of a K and a V tile; lane -> row RPP piece + lane / RCH, stored
+    // chunk lane % RCH
     const char *   kbase = a.k + hk * a.knb2 + bk * a.knb3;
     const char *   vbase = a.v + hk * a.vnb2 + bk * a.vnb3;
     const uint32_t sbase = (uint32_t) (uintptr_t) (__attribute__((address_space(3))) char *) smem;
-    const int      drow = lane >> 4, dpc = lane & 15;
+    const int      drow = lane / RCH, dpc = lane % RCH;
+    // 16-byte chunk swizzle of K row r: 16 consecutive rows at one chunk hit 64 banks
+    auto kswz = [](int r) { return D == 128 ? r & 15 : (r >> 1) & 7; };
     auto dma_k = [&](int j) {
 #pragma unroll
         for (int i = 0; i < PPW; i++) {
-            const int piece = PPW * wave + i, r = 4 * piece + drow;
+            const int piece = PPW * wave + i, r = RPP * piece + drow;
             const int key   = min(j * FA_BK + r, a.nkv - 1);  // rows past the end repeat the last key (masked below)
-            fa_dma16(kbase + (int64_t) key * a.knb1 + ((dpc ^ (r & 15)) << 4),
+            fa_dma16(kbase + (int64_t) key * a.knb1 + ((dpc ^ kswz(r)) << 4),
                      sbase + (j & (KR - 1)) * TILE + piece * 1024);
         }
     };
     auto dma_v = [&](int j) {
 #pragma unroll
         for (int i = 0; i < PPW; i++) {
-            const int piece = PPW * wave + i, r = 4 * piece + drow;
-            const int key   = min(j * FA_BK + r, a.nkv - 1);
-            fa_dma16(vbase + (int64_t) key * a.vnb1 + ((dpc ^ (2 * (r & 3))) << 4),
-                     sbase + (KR + (j & (KR - 1))) * TILE + piece * 1024);
+            const int piece = PPW * wave + i, r = RPP * piece + drow;
+            const int key   = j * FA_BK + r;
+            // keys past the end read zeros: p = 0 times a last row holding inf would be NaN
+            const char * row = key < a.nkv ? vbase + (int64_t) key * a.vnb1 + ((dpc ^ (2 * (r & 3))) << 4)
+                                           : (const char *) fa_zeros;
+            fa_dma16(row, sbase + (KR + (j & (KR - 1))) * TILE + piece * 1024);
         }
     };
     // K operand of k-step kk: row lq of the 32-key unit, logical chunk 2 kk + hh
     uint32_t ka[NQK];
 #pragma unroll
     for (int kk = 0; kk < NQK; kk++) {
-        ka[kk] = lq * 256 + (((2 * kk + hh) ^ (lq & 15)) << 4);
+        ka[kk] = lq * RB + (((2 * kk + hh) ^ kswz(lq)) << 4);
     }
     // V^T operand: source lane (tg, tj, tq) of a transposed read addresses
     // V[key0 + 4 (tg / 2) + tj][32 db + 16 (tg & 1) + 4 tq]; the V swizzle
@@ -550,20 +568,23 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
     const int      tg = lane >> 4, tj = (lane >> 2) & 3, tq = lane & 3;
     const int      vx = (tj >> 1) * 64;
     const uint32_t vlane =
-        (4 * (tg >> 1) + tj) * 256 + 16 * ((2 * (tg & 1) + (tq >> 1)) ^ (2 * (tj & 1))) + 8 * (tq & 1);
+        (4 * (tg >> 1) + tj) * RB + 16 * ((2 * (tg & 1) + (tq >> 1)) ^ (2 * (tj & 1))) + 8 * (tq & 1);
     const uint32_t vb[2] = { vlane + vx, vlane - vx };
-    auto qk_op = [&](int u, int kk) -> half8_t {
-        const char * kt = smem + ((u >> 1) & (KR - 1)) * TILE;
-        return *(const half8_t *) (kt + ka[kk] + (u & 1) * 8192);
+    // QK step i of a unit: key block c = i % UK (32 keys), 16-dim step i / UK
+    auto qk_op = [&](int u, int i) -> half8_t {
+        const int    sub = UK == 2 ? i % UK : u & 1, tile = UK == 2 ? u : u >> 1;
+        const char * kt  = smem + (tile & (KR - 1)) * TILE;
+        return *(const half8_t *) (kt + ka[i / UK] + sub * (TILE / 2));
     };
-    // PV step i of a unit: key half t = i / 4 (16 keys), output block db = i % 4
+    // PV step i of a unit: key group t = i / NDB (16 keys), output block db = i % NDB
     auto pv_op = [&](int u, int i) -> half8_t {
-        const uint32_t vt = sbase + (KR + ((u >> 1) & (KR - 1))) * TILE;
-        const int      t = i >> 2, db = i & 3;
+        const int      tile = UK == 2 ? u : u >> 1, sub = UK == 2 ? 0 : u & 1;
+        const uint32_t vt   = sbase + (KR + (tile & (KR - 1))) * TILE;
+        const int      t = i / NDB, db = i % NDB;
         half8_t        av;
 #pragma unroll
         for (int hf = 0; hf < 2; hf++) {
-            const uint32_t ad = vt + vb[db & 1] + ((u & 1) * 32 + 16 * t + 8 * hf) * 256 + 64 * db;
+            const uint32_t ad = vt + vb[db & 1] + (sub * 32 + 16 * t + 8 * hf) * RB + 64 * db;
             const half4_t  x  = __builtin_bit_cast(
                 half4_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_t *) (uintptr_t) ad));
 #pragma unroll
@@ -580,15 +601,19 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
         zero16[r] = 0.0f;
         negm[r]   = 0.0f;
     }
-    float16_t sc, sn;         // s - m of unit u (softmax input) and of unit u + 1 (being computed)
-    half8_t   pp[2], pn[2];   // P of unit u - 1 (PV input) and of unit u (softmax output)
-    float     m_sn = 0.0f;    // the m that sn was computed against
+    // scores s - m of two units (softmax input, the next unit's being computed)
+    // and P of two units (softmax output, PV input of the next): the units
+    // alternate between them, so nothing is copied
+    float16_t sA[UK], sB[UK];
+    half8_t   pX[2 * UK], pY[2 * UK];
+    float     m_sn = 0.0f;    // the m that the scores being computed are against
     const half2_t ones2 = { (_Float16) 1.0f, (_Float16) 1.0f };
-    auto exp_pack = [&](float & rs) {
+    auto exp_pack = [&](float & rs, float16_t (&sc)[UK], half8_t (&pn)[2 * UK]) {
         rs = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 16; r += 2) {
-            const half2_t pk = { (_Float16) __builtin_amdgcn_exp2f(sc[r]), (_Float16) __builtin_amdgcn_exp2f(sc[r + 1]) };
+        for (int r = 0; r < 16 * UK; r += 2) {
+            const half2_t pk = { (_Float16) __builtin_amdgcn_exp2f(sc[r >> 4][r & 15]),
+                                 (_Float16) __builtin_amdgcn_exp2f(sc[r >> 4][(r & 15) + 1]) };
             rs                        = __builtin_amdgcn_fdot2(pk, ones2, rs, false);
             pn[r >> 3][r & 7]         = pk[0];
             pn[r >> 3][(r & 7) + 1]   = pk[1];
@@ -596,11 +621,11 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
     };
     // move m to the row max (first unit: exactly; later: upwards only),
     // rescale O and l, redo the unit's p
-    auto slow = [&](float & rs, bool first_unit) {
+    auto slow = [&](float & rs, bool first_unit, float16_t (&sc)[UK], half8_t (&pn)[2 * UK]) {
         float mx = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            mx = fmaxf(mx, sc[r]);
+        for (int r = 0; r < 16 * UK; r++) {
+            mx = fmaxf(mx, sc[r >> 4][r & 15]);
         }
         mx = max_xor32(mx);
         // first: nothing visible accumulated yet (O and l zero), m goes to
@@ -623,8 +648,8 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
                 }
             }
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                sc[r] -= d;
+            for (int r = 0; r < 16 * UK; r++) {
+                sc[r >> 4][r & 15] -= d;
             }
             m += d;
 #pragma unroll
@@ -632,73 +657,80 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
                 negm[r] = -m;
             }
         }
-        exp_pack(rs);
+        exp_pack(rs, sc, pn);
     };
     // unit u: softmax(u) (SM), QK(u + US) (QK), PV(u - US) (PV); which parts
     // are present is a compile-time choice, so the steady-state unit is
     // branch-free and the compiler interleaves its VALU work with the MFMAs
-    auto unit = [&](int u, auto QKc, auto PVc, auto SMc) {
+    auto unit = [&](int u, float16_t (&sc)[UK], float16_t (&sn)[UK], half8_t (&pp)[2 * UK], half8_t (&pn)[2 * UK],
+                    auto QKc, auto PVc, auto SMc) {
         constexpr bool do_qk = decltype(QKc)::value, do_pv = decltype(PVc)::value, do_sm = decltype(SMc)::value;
         if constexpr (do_sm) {
-            const int k0 = u * 32;
-            if (k0 + 32 > a.nkv) {  // the last, partial unit
+            const int k0 = u * UB;
+            if (k0 + UB > a.nkv) {  // the last, partial unit
 #pragma unroll
-                for (int r = 0; r < 16; r++) {
+                for (int r = 0; r < 16 * UK; r++) {
                     if (k0 + 8 * (r / 4) + 4 * hh + (r % 4) >= a.nkv) {
-                        sc[r] = -INFINITY;
+                        sc[r >> 4][r & 15] = -INFINITY;
                     }
                 }
             }
         }
         const float m_used = m;
         float       rs     = 0.0f;
-        // operands three MFMA steps ahead; the scheduling barrier keeps each
+        // operands PF MFMA steps ahead; the scheduling barrier keeps each
         // step's LDS reads above it (left alone, the scheduler sank them to
         // just before their MFMA, reusing one register set, so every MFMA
-        // waited out a whole LDS read).  Masked: nothing crosses it (the
-        // lone long-row waves of a causal workgroup: 50.1 -> 44.8 us at B = 2,
-        // S = 1024); unmasked: ALU, MFMA and transcendental work may
-        // (the DiT shape: 295 -> 291 us)
-        half8_t     av[4], ak[4];
+        // waited out a whole LDS read).  Four waves: nothing crosses it
+        // (causal, B = 2, S = 1024: 50.1 -> 44.8 us; S = 690, D = 64, B = 2:
+        // 19.8 -> 18.8 us) and two steps do (three spill in the masked form:
+        // 39.2 against 38.8 us).  Eight waves, three steps: ALU, MFMA and
+        // transcendental work may (S = 4096: 278 -> 273 us)
+        constexpr int PF = NW == 8 ? 3 : 2;
+        half8_t       av[PF + 1], ak[PF + 1];
         if constexpr (do_pv) {
-            av[0] = pv_op(u - US, 0);
-            av[1] = pv_op(u - US, 1);
-            av[2] = pv_op(u - US, 2);
+#pragma unroll
+            for (int i = 0; i < PF; i++) {
+                av[i] = pv_op(u - US, i);
+            }
         }
         if constexpr (do_qk) {
-            ak[0] = qk_op(u + US, 0);
-            ak[1] = qk_op(u + US, 1);
-            ak[2] = qk_op(u + US, 2);
+#pragma unroll
+            for (int i = 0; i < PF; i++) {
+                ak[i] = qk_op(u + US, i);
+            }
         }
 #pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (i + 3 < 8) {
+        for (int i = 0; i < NS; i++) {
+            if (i + PF < NS) {
                 if constexpr (do_pv) {
-                    av[(i + 3) % 4] = pv_op(u - US, i + 3);
+                    av[(i + PF) % (PF + 1)] = pv_op(u - US, i + PF);
                 }
                 if constexpr (do_qk) {
-                    ak[(i + 3) % 4] = qk_op(u + US, i + 3);
+                    ak[(i + PF) % (PF + 1)] = qk_op(u + US, i + PF);
                 }
             }
-            __builtin_amdgcn_sched_barrier(MASK ? 0 : 0x040F);
+            __builtin_amdgcn_sched_barrier(NW == 4 ? 0 : 0x040F);
             if constexpr (do_pv) {
-                oacc[i & 3] = mfma32(av[i % 4], pp[i >> 2], oacc[i & 3]);
+                oacc[i % NDB] = mfma32(av[i % (PF + 1)], pp[i / NDB], oacc[i % NDB]);
             }
             if constexpr (do_qk) {
-                sn = mfma32(ak[i % 4], qreg[i], i == 0 ? negm : sn);
+                sn[i % UK] = mfma32(ak[i % (PF + 1)], qreg[i / UK], i < UK ? negm : sn[i % UK]);
             }
             if constexpr (do_sm) {
-                const int     r  = 2 * i;
-                const half2_t pk = { (_Float16) __builtin_amdgcn_exp2f(sc[r]),
-                                     (_Float16) __builtin_amdgcn_exp2f(sc[r + 1]) };
-                rs                      = __builtin_amdgcn_fdot2(pk, ones2, rs, false);
-                pn[r >> 3][r & 7]       = pk[0];
-                pn[r >> 3][(r & 7) + 1] = pk[1];
+#pragma unroll
+                for (int r = 16 / NQK * i; r < 16 / NQK * (i + 1); r += 2) {
+                    const half2_t pk = { (_Float16) __builtin_amdgcn_exp2f(sc[r >> 4][r & 15]),
+                                         (_Float16) __builtin_amdgcn_exp2f(sc[r >> 4][(r & 15) + 1]) };
+                    rs                      = __builtin_amdgcn_fdot2(pk, ones2, rs, false);
+                    pn[r >> 3][r & 7]       = pk[0];
+                    pn[r >> 3][(r & 7) + 1] = pk[1];
+                }
             }
         }
         if constexpr (do_sm) {
             if ((MASK ? __any(!mset) : u == 0) || __any(rs > 16384.0f)) {
-                slow(rs, u == 0);
+                slow(rs, u == 0, sc, pn);
             }
             l += rs;
         }
@@ -709,7 +741,7 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
     // DMA group g (g >= -KR / 2): K tile g + KR and V tile g + KR - 1, each
     // PPW loads per wave when the tile exists; the groups before 0 go out
     // after the prologue, group j after the barrier that follows unit 2 j
-    auto group_loads = [&](int g) { return PPW * (g + KR < n) + PPW * (g + KR - 1 < n); };
+    auto group_tiles = [&](int g) { return (g + KR < n) + (g + KR - 1 < n); };
     auto issue_group = [&](int g) {
         if (g + KR < n) {
             dma_k(g + KR);
@@ -719,36 +751,37 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
         }
     };
     // after unit u: sn becomes the next softmax input (shifted if m moved
-    // since it was computed); after an even unit 2 j: the wait for K tile
+    // since it was computed); then, once per tile, the wait, the barrier and
+    // the next DMA group.  UK = 1, after an even unit 2 j: the wait for K tile
     // j + 1 and V tile j (group j - 3: only the loads of groups j - 2 and
-    // j - 1 may still be in flight), the barrier, then group j: K tile j + 4
-    // into the buffer of K tile j (last read in unit 2 j), V tile j + 3 into
-    // that of V tile j - 1 (last read in unit 2 j)
-    auto after = [&](int u) {
-        sc = sn;
+    // j - 1 may still be in flight), then group j: K tile j + 4 into the
+    // buffer of K tile j (last read in unit 2 j), V tile j + 3 into that of V
+    // tile j - 1 (last read in unit 2 j).  UK = 2, after unit j: the wait for
+    // K tile j + 2 and V tile j (the first half of group j - 2: its V tile
+    // and group j - 1 may be in flight), then group j: K tile j was last read
+    // in unit j - 1, V tile j - 1 in unit j
+    auto after = [&](int u, float16_t (&sc)[UK]) {
         if (__any(m_sn != m)) {
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                sc[r] += m_sn - m;
+            for (int r = 0; r < 16 * UK; r++) {
+                sc[r >> 4][r & 15] += m_sn - m;
             }
         }
         if (mask_need(u + US) && u + US < nu) {
-            mask_apply(sc);
+            mask_apply(sc[0]);
         }
-        pp[0] = pn[0];
-        pp[1] = pn[1];
-        if ((u & 1) == 0) {
-            const int j = u >> 1;
+        if (UK == 2 || (u & 1) == 0) {
+            const int j = UK == 2 ? u : u >> 1;
             if constexpr (KR == 2) {
                 // K tile j + 1 and V tile j: group j - 1, the last one issued
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             } else {
-                switch (group_loads(j - 2) + group_loads(j - 1)) {
+                switch ((UK == 2 ? (j - 2 + KR - 1 < n) : group_tiles(j - 2)) + group_tiles(j - 1)) {
                     case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
-                    case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
-                    case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
-                    case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
-                    default: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
+                    case 1: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PPW) : "memory"); break;
+                    case 2: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PPW) : "memory"); break;
+                    case 3: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * PPW) : "memory"); break;
+                    default: asm volatile("s_waitcnt vmcnt(%0)" ::"n"(4 * PPW) : "memory"); break;
                 }
             }
             asm volatile("s_barrier" ::: "memory");
@@ -777,14 +810,17 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
         issue_group(-2);
     }
     issue_group(-1);
-    sc = zero16;
+#pragma unroll
+    for (int c = 0; c < UK; c++) {
+        sA[c] = zero16;
+    }
     if (nk > 0) {
 #pragma unroll
-        for (int kk = 0; kk < NQK; kk++) {
-            sc = mfma32(qk_op(u0, kk), qreg[kk], sc);
+        for (int i = 0; i < NS; i++) {
+            sA[i % UK] = mfma32(qk_op(u0, i), qreg[i / UK], sA[i % UK]);
         }
         if (mask_need(u0)) {
-            mask_apply(sc);
+            mask_apply(sA[0]);
         }
     }
     using T_ = std::integral_constant<bool, true>;
@@ -796,33 +832,54 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
     // drained PV reads a V tile that is restaged after the next step at the
     // earliest.
     if (nk > 0) {
-        if (nk > 1 && mask_need(u0 + US)) {
-            mask_load(u0 + US);
-        }
-        if (nk > 1) {
-            unit(u0, T_{}, F_{}, T_{});
-        } else {
-            unit(u0, F_{}, F_{}, T_{});
-        }
-        after(u0);
-        for (int i = 1; i + 1 < nk; i++) {
-            const int u = u0 + i * US;
-            if (mask_need(u + US)) {
-                mask_load(u + US);
+        auto prefetch_mask = [&](int i) {
+            if (i < nk && mask_need(u0 + i * US)) {
+                mask_load(u0 + i * US);
             }
-            unit(u, T_{}, T_{}, T_{});
-            after(u);
+        };
+        prefetch_mask(1);
+        if (nk > 1) {
+            unit(u0, sA, sB, pX, pY, T_{}, F_{}, T_{});
+        } else {
+            unit(u0, sA, sB, pX, pY, F_{}, F_{}, T_{});
+        }
+        after(u0, sB);
+        int i = 1;  // here: unit i's scores in sB, P of unit i - 1 in pY
+        for (; i + 2 < nk; i += 2) {
+            prefetch_mask(i + 1);
+            unit(u0 + i * US, sB, sA, pY, pX, T_{}, T_{}, T_{});
+            after(u0 + i * US, sA);
+            prefetch_mask(i + 2);
+            unit(u0 + (i + 1) * US, sA, sB, pX, pY, T_{}, T_{}, T_{});
+            after(u0 + (i + 1) * US, sB);
+        }
+        auto p_to_y = [&]() {
+#pragma unroll
+            for (int t = 0; t < 2 * UK; t++) {
+                pY[t] = pX[t];
+            }
+        };
+        if (i + 1 < nk) {
+            prefetch_mask(i + 1);
+            unit(u0 + i * US, sB, sA, pY, pX, T_{}, T_{}, T_{});
+            after(u0 + i * US, sA);
+#pragma unroll
+            for (int c = 0; c < UK; c++) {
+                sB[c] = sA[c];
+            }
+            p_to_y();
         }
         if (nk > 1) {
             const int u = u0 + (nk - 1) * US;
-            unit(u, F_{}, T_{}, T_{});
-            after(u);
+            unit(u, sB, sA, pY, pX, F_{}, T_{}, T_{});
+            after(u, sB);
+            p_to_y();
         }
-        unit(u0 + nk * US, F_{}, T_{}, F_{});
+        unit(u0 + nk * US, sB, sA, pY, pX, F_{}, T_{}, F_{});
     }
     if constexpr (MASK) {
         for (int u = nu; u < nu_wg; u++) {
-            after(u);
+            after(u, sB);
         }
     }
 
@@ -844,22 +901,28 @@ __global__ __launch_bounds__(NW * 64, 2) void k_fa_dma(FaArgs a, const int * __r
 }
 
 // k_fa_dma's preconditions: 16-byte aligned Q rows (float4 loads) and K / V
-// rows (16-byte DMA), D = 128, and at least one workgroup of 256 rows per CU
-// (MMHIP_DISABLE_FA_DMA=1 takes the register-staged kernel instead)
-constexpr size_t FA_DMA_LDS  = 8 * FA_BK * 256;  // K and V rings of 4 tiles
-constexpr size_t FA_DMA_LDS2 = 4 * FA_BK * 256;  // K and V rings of 2 tiles (two workgroups per CU)
-
-static int fa_dma_qtiles(const FaArgs & a) {
-    return a.mask ? (a.nq + 127) / 128 : (a.nq + 255) / 256;
-}
-
+// rows (16-byte DMA) (MMHIP_DISABLE_FA_DMA=1 takes the register-staged kernel
+// instead)
 static bool fa_dma_ok(const FaArgs & a, int D) {
     auto al16 = [](int64_t v) { return (v & 15) == 0; };
-    const int64_t tiles = (int64_t) fa_dma_qtiles(a) * a.Hq * a.B;
-    return D == 128 && !getenv("MMHIP_DISABLE_FA_DMA") && tiles >= 256 && a.nkv >= 1 &&
+    const bool shape = a.mask ? D == 128 && (int64_t) ((a.nq + 127) / 128) * a.Hq * a.B >= 256 : D == 64 || D == 128;
+    return shape && !getenv("MMHIP_DISABLE_FA_DMA") && a.nkv >= 1 &&
            al16((int64_t) (uintptr_t) a.q) && al16(a.qnb1) &&
            al16(a.qnb2) && al16(a.qnb3) && al16((int64_t) (uintptr_t) a.k) && al16(a.knb1) && al16(a.knb2) &&
            al16(a.knb3) && al16((int64_t) (uintptr_t) a.v) && al16(a.vnb1) && al16(a.vnb2) && al16(a.vnb3);
+}
+
+template <bool MASK, int D, int NW, int KR, int UK>
+static int launch_fa_dma(const FaArgs & a, const int * row_end, const int * zero_end, float * out, hipStream_t stream) {
+    const int        nqt  = (a.nq + 32 * NW - 1) / (32 * NW);
+    constexpr size_t lds  = (size_t) 2 * KR * FA_BK * 2 * D;  // K and V rings of KR tiles
+    auto             kern = k_fa_dma<MASK, D, NW, KR, UK>;
+    if (!ensure_lds_limit((const void *) kern, lds)) {
+        return set_error(MMHIP_ERR_HIP, "flash_attn dma: cannot raise the LDS limit");
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned) (nqt * a.Hq * a.B)), dim3(NW * 64), lds, stream, a, row_end, zero_end, nqt,
+                       out);
+    return check_launch("flash_attn dma");
 }
 
 // Mask prepass: for every mask plane (mask batch x mask head) and query row,
@@ -961,22 +1024,16 @@ int fa_mfma(const FaArgs & a, int D, float * out, void * ws, size_t ws_bytes, hi
         }
     }
     if (fa_dma_ok(a, D)) {
-        const int    nqt = fa_dma_qtiles(a);
-        const size_t lds = FA_DMA_LDS;
         if (a.mask) {
-            if (!ensure_lds_limit((const void *) k_fa_dma<true, 4, 2>, FA_DMA_LDS2)) {
-                return set_error(MMHIP_ERR_HIP, "flash_attn dma: cannot raise the LDS limit");
-            }
-            hipLaunchKernelGGL((k_fa_dma<true, 4, 2>), dim3((unsigned) (nqt * a.Hq * a.B)), dim3(256), FA_DMA_LDS2,
-                               stream, a, row_end, zero_end, nqt, out);
-        } else {
-            if (!ensure_lds_limit((const void *) k_fa_dma<false>, lds)) {
-                return set_error(MMHIP_ERR_HIP, "flash_attn dma: cannot raise the LDS limit");
-            }
-            hipLaunchKernelGGL(k_fa_dma<false>, dim3((unsigned) (nqt * a.Hq * a.B)), dim3(512), lds, stream, a,
-                               nullptr, nullptr, nqt, out);
+            return launch_fa_dma<true, 128, 4, 2, 1>(a, row_end, zero_end, out, stream);
         }
-    } else if (D == 128) {
+        if (D == 64) {
+            return launch_fa_dma<false, 64, 4, 4, 2>(a, nullptr, nullptr, out, stream);
+        }
+        return NW == 8 ? launch_fa_dma<false, 128, 8, 4, 1>(a, nullptr, nullptr, out, stream)
+                       : launch_fa_dma<false, 128, 4, 4, 1>(a, nullptr, nullptr, out, stream);
+    }
+    if (D == 128) {
         NW == 8 ? launch_fa_mfma<128, 8>(a, row_end, zero_end, n_qtiles, out, stream)
                 : launch_fa_mfma<128, 4>(a, row_end, zero_end, n_qtiles, out, stream);
     } else if (D == 64) {
