@@ -211,6 +211,16 @@ int mmhip_rms_norm_mul_mat_supported(int type, int64_t N, int64_t K, int64_t M);
 int mmhip_rms_norm_mul_mat(int type, const void * W, int64_t N, int64_t K, int64_t w_row_stride, const float * x,
                            int64_t ldx, int64_t M, const float * norm_w, float eps, float * xn_out, const float * r,
                            int64_t ldr, float * y, int64_t ldy, void * stream);
+
+/* Two mmhip_rms_norm_mul_mat of the same rows in one launch, each with its own
+ * arithmetic: a Q4_K / Q5_K matrix and a Q6_K one (the decode step's fused Q
+ * and K rows beside the V projection that a Q4_K_M / Q5_K_M file keeps in
+ * Q6_K, src/qwen3-lm.h:386-399).  K = 4096, M = 1 or 2. */
+int mmhip_rms_norm_mul_mat_pair_supported(int type, int64_t N, int type2, int64_t N2, int64_t K, int64_t M);
+int mmhip_rms_norm_mul_mat_pair(int type, const void * W, int64_t N, int64_t w_row_stride, float * y, int64_t ldy,
+                                int type2, const void * W2, int64_t N2, int64_t w2_row_stride, float * y2, int64_t ldy2,
+                                int64_t K, const float * x, int64_t ldx, int64_t M, const float * norm_w, float eps,
+                                void * stream);
 /* The GEMV that follows a SwiGLU, with the SwiGLU in its prologue: the
  * GGML_OP_GLU (swiglu / swiglu_split, src/qwen3-enc.h:106-113) feeding the
  * MLP down GGML_OP_MUL_MAT (src/qwen3-enc.h:114) whose residual GGML_OP_ADD

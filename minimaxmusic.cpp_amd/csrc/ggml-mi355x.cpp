@@ -1021,6 +1021,7 @@ struct plan_step {
     int                  glu_epi  = -1;  // MM / GEMM: the SWIGLU node computed in the GEMV's / GEMM's epilogue
     int                  glu_swapped = 0;  // GEMM: the gate rows are the first half
     int                  multi[2]    = { -1, -1 };  // GEMM / MM: further MUL_MATs of the same activations in this launch
+    int                  pair     = -1;  // MM: a second normed MUL_MAT of the same rows in this launch
     int                  mm       = -1;  // GEMM: the MUL_MAT node
     int                  bias     = -1;  // GEMM: the bias ADD node / LN: the ADD of the LayerNorm bias
     int                  bias_src = -1;  // index 0/1 of that ADD's vector operand
@@ -2193,6 +2194,48 @@ graph_plan build_plan(struct ggml_cgraph * g) {
         }
     }
     plan.steps.swap(merged);
+    // neighbouring normed GEMVs of the same rows, one Q4_K / Q5_K and one Q6_K
+    // (Q and K rows, and a V projection of another type): one launch, the
+    // Q6_K one as the step's `pair`
+    if (getenv("GGML_MI355X_DISABLE_GEMV_PAIR") == nullptr && !no_fuse) {
+        for (size_t x = 0; x < plan.steps.size(); x++) {
+            size_t y = x + 1;
+            while (y < plan.steps.size() && plan.steps[y].kind == ST_NODE &&
+                   is_noop(ggml_graph_node(g, plan.steps[y].node)->op)) {
+                y++;
+            }
+            if (y >= plan.steps.size()) {
+                break;
+            }
+            const plan_step *          s[2] = { &plan.steps[x], &plan.steps[y] };
+            const struct ggml_tensor * m[2];
+            bool                       ok = true;
+            for (int k = 0; k < 2 && ok; k++) {
+                ok   = s[k]->kind == ST_MM && s[k]->norm >= 0 && s[k]->add < 0 && s[k]->glu < 0 && s[k]->glu_epi < 0 &&
+                     s[k]->multi[0] < 0 && s[k]->pair < 0;
+                m[k] = ok ? ggml_graph_node(g, s[k]->node) : nullptr;
+            }
+            if (!ok || s[0]->norm != s[1]->norm || s[0]->norm_mul != s[1]->norm_mul) {
+                continue;
+            }
+            const int                  a = m[0]->src[0]->type == GGML_TYPE_Q6_K ? 1 : 0;
+            const struct ggml_tensor * w = m[a]->src[0];
+            const struct ggml_tensor * v = m[1 - a]->src[0];
+            const struct ggml_tensor * xr = ggml_graph_node(g, s[0]->norm)->src[0];
+            const int64_t              M  = m[0]->src[1]->ne[1] * m[0]->src[1]->ne[2] * m[0]->src[1]->ne[3];
+            if (w->ne[0] != v->ne[0] ||
+                !mmhip_rms_norm_mul_mat_pair_supported(w->type, w->ne[1], v->type, v->ne[1], w->ne[0], M) ||
+                overlaps(m[0], m[1]) || overlaps(m[0], xr) || overlaps(m[1], xr) || overlaps(m[a], v) ||
+                overlaps(m[1 - a], w)) {
+                continue;
+            }
+            plan_step f = *s[a];
+            f.pair      = s[1 - a]->node;
+            // at the later one's place: nothing between them reads the first
+            plan.steps[y] = f;
+            plan.steps.erase(plan.steps.begin() + (long) x);
+        }
+    }
     // a HEAD step of Q, K and V chains followed (past views only) by the
     // decode attention they feed: one launch, the chains in its prologue
     if (getenv("GGML_MI355X_DISABLE_FA_HEAD") == nullptr && !no_fuse) {
@@ -2465,6 +2508,15 @@ int run_step(mi_backend * c, struct ggml_cgraph * g, const plan_step & st, char 
                                                     (int64_t) (xr->nb[1] / 4), M, (const float *) nwt->data, eps,
                                                     gn->op_params[1] != 0, slot + st.slot_out,
                                                     st.write_f32 ? (float *) gn->data : nullptr, s);
+                    break;
+                }
+                if (st.pair >= 0) {
+                    const struct ggml_tensor * m2 = ggml_graph_node(g, st.pair);
+                    const struct ggml_tensor * w2 = m2->src[0];
+                    rc = mmhip_rms_norm_mul_mat_pair(w->type, w->data, N, (int64_t) w->nb[1], (float *) n->data, N,
+                                                     w2->type, w2->data, w2->ne[1], (int64_t) w2->nb[1],
+                                                     (float *) m2->data, w2->ne[1], K, (const float *) xr->data,
+                                                     (int64_t) (xr->nb[1] / 4), M, (const float *) nwt->data, eps, s);
                     break;
                 }
                 rc = mmhip_rms_norm_mul_mat(w->type, w->data, N, K, (int64_t) w->nb[1], (const float *) xr->data,

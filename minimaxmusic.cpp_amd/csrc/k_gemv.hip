@@ -605,7 +605,7 @@ struct Pg6Act {
 };
 
 template <int NC, int CH, int PRO>
-__global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q6_K_pro(PgArgs a, Pg6Act xa) {
+__device__ __forceinline__ void gemv_q6_K_wg(const PgArgs & a, const Pg6Act & xa, int wg, int wgs) {
     constexpr int  MAXK = 4096 * CH;
     constexpr int  J    = MAXK / (256 * PG_WAVES);
     constexpr bool DB   = CH == 1;
@@ -616,8 +616,8 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q6_K_pro(PgArgs a, Pg6Ac
     __shared__ double  s_ss[NC][PG_WAVES];
     const int     lane  = threadIdx.x & 63;
     const int     wv    = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t gw    = (int64_t) blockIdx.x * PG_WAVES + wv;
-    const int64_t TW    = (int64_t) gridDim.x * PG_WAVES;
+    const int64_t gw    = (int64_t) wg * PG_WAVES + wv;
+    const int64_t TW    = (int64_t) wgs * PG_WAVES;
     const int     K     = a.K;
     const int     units = K / 64;
     // 1. activations (or the quantised rows), then the first weight rows
@@ -746,6 +746,11 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q6_K_pro(PgArgs a, Pg6Ac
     }
 }
 
+template <int NC, int CH, int PRO>
+__global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q6_K_pro(PgArgs a, Pg6Act xa) {
+    gemv_q6_K_wg<NC, CH, PRO>(a, xa, (int) blockIdx.x, (int) gridDim.x);
+}
+
 // Persistent Q4_K / Q5_K GEMVs (M <= 2, K = 4096 CH) with the structure of
 // k_gemv_q6_K_pro: PRO_NORM (the RMS norm and the Q8_K quantisation of the
 // activation rows in the prologue) or PRO_NONE (a copy of quantised Q8_K
@@ -871,7 +876,7 @@ __device__ __forceinline__ void pg5_col(const int4_t (&q)[4], const int (&sc)[4]
 }
 
 template <int NC, int CH, int PRO, bool Q5>
-__global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q45_K_pro(PgArgs a, Pg6Act xa) {
+__device__ __forceinline__ void gemv_q45_K_wg(const PgArgs & a, const Pg6Act & xa, int wg, int wgs) {
     static_assert(PRO == PRO_NORM || PRO == PRO_NONE, "Q4_K / Q5_K: norm or quantised-row prologue");
     constexpr int  MAXK = 4096 * CH;
     constexpr int  J    = MAXK / (256 * PG_WAVES);
@@ -882,8 +887,8 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q45_K_pro(PgArgs a, Pg6A
     __shared__ double  s_ss[NC][PG_WAVES];
     const int     lane = threadIdx.x & 63;
     const int     wv   = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t gw   = (int64_t) blockIdx.x * PG_WAVES + wv;
-    const int64_t TW   = (int64_t) gridDim.x * PG_WAVES;
+    const int64_t gw   = (int64_t) wg * PG_WAVES + wv;
+    const int64_t TW   = (int64_t) wgs * PG_WAVES;
     const int     K    = a.K;
     // 1. activations (or the quantised rows), then the first weight rows
     float4_t xv[J][NC], xw[J][1];
@@ -993,6 +998,25 @@ __global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q45_K_pro(PgArgs a, Pg6A
             }
             pg5_load<CH, Q5>(ba, a, it * TW + gw, lane);
         }
+    }
+}
+
+template <int NC, int CH, int PRO, bool Q5>
+__global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q45_K_pro(PgArgs a, Pg6Act xa) {
+    gemv_q45_K_wg<NC, CH, PRO, Q5>(a, xa, (int) blockIdx.x, (int) gridDim.x);
+}
+
+// A Q4_K / Q5_K matrix (a, the first na workgroups) and a Q6_K one (v, the
+// rest) on the same RMS-normed rows (the decode step's fused Q and K rows and
+// the V projection a Q4_K_M / Q5_K_M file keeps in Q6_K): both are latency
+// (norm prologue, then one or two rows a wave), so they run beside each other
+// on different CUs instead of one after the other.
+template <int NC, bool Q5>
+__global__ __launch_bounds__(64 * PG_WAVES) void k_gemv_q45_q6_norm(PgArgs a, PgArgs v, int na) {
+    if ((int) blockIdx.x < na) {
+        gemv_q45_K_wg<NC, 1, PRO_NORM, Q5>(a, Pg6Act{}, (int) blockIdx.x, na);
+    } else {
+        gemv_q6_K_wg<NC, 1, PRO_NORM>(v, Pg6Act{}, (int) blockIdx.x - na, (int) gridDim.x - na);
     }
 }
 
@@ -2543,6 +2567,44 @@ extern "C" int mmhip_rms_norm_mul_mat(int type, const void * W, int64_t N, int64
     const PgArgs a{ (const uint8_t *) W, N, (int) K, w_row_stride, x, ldx, nullptr, 0, norm_w, eps, xn_out, y, ldy,
                     res, ldr, 1 };
     return dispatch_pro<PRO_NORM>(type, a, M, (hipStream_t) stream, "rms_norm_mul_mat");
+}
+
+extern "C" int mmhip_rms_norm_mul_mat_pair_supported(int type, int64_t N, int type2, int64_t N2, int64_t K, int64_t M) {
+    return (type == TYPE_Q4_K || type == TYPE_Q5_K) && type2 == TYPE_Q6_K && pro_supported(PRO_NORM, type, N, K, M) &&
+           pro_supported(PRO_NORM, type2, N2, K, M) && N <= (1 << 20) && N2 <= (1 << 20);
+}
+
+extern "C" int mmhip_rms_norm_mul_mat_pair(int type, const void * W, int64_t N, int64_t w_row_stride, float * y,
+                                           int64_t ldy, int type2, const void * W2, int64_t N2,
+                                           int64_t w2_row_stride, float * y2, int64_t ldy2, int64_t K, const float * x,
+                                           int64_t ldx, int64_t M, const float * norm_w, float eps, void * stream) {
+    MMHIP_API_BEGIN();
+    if (!mmhip_rms_norm_mul_mat_pair_supported(type, N, type2, N2, K, M)) {
+        return set_error(MMHIP_ERR_UNSUPPORTED, "rms_norm_mul_mat_pair: types %d %d N=%lld %lld K=%lld M=%lld", type,
+                         type2, (long long) N, (long long) N2, (long long) K, (long long) M);
+    }
+    if (!W || !W2 || !x || !norm_w || !y || !y2 || ldx < K || ldy < N || ldy2 < N2 ||
+        !gemv_supported(type, N, K, w_row_stride, W) || !gemv_supported(type2, N2, K, w2_row_stride, W2) ||
+        !pro_rows_ok(type, w_row_stride, W) || !pro_rows_ok(type2, w2_row_stride, W2) ||
+        ((uintptr_t) x | (uintptr_t) norm_w) % 16 != 0 || (ldx % 4) != 0) {
+        return set_error(MMHIP_ERR_INVALID, "rms_norm_mul_mat_pair: bad arguments / alignment");
+    }
+    // each matrix's rows split over workgroups as in its own launch
+    auto split = [](PgArgs & a) {
+        const int64_t need = (a.N + PG_WAVES - 1) / PG_WAVES;
+        a.nit              = (int) ((need + pg_cus() - 1) / pg_cus());
+        return (need + a.nit - 1) / a.nit;
+    };
+    PgArgs a{ (const uint8_t *) W, N, (int) K, w_row_stride, x, ldx, nullptr, 0, norm_w, eps, nullptr, y, ldy, nullptr, 0,
+              1 };
+    PgArgs v{ (const uint8_t *) W2, N2, (int) K, w2_row_stride, x, ldx, nullptr, 0, norm_w, eps, nullptr, y2, ldy2,
+              nullptr, 0, 1 };
+    const int64_t na = split(a), nv = split(v);
+    const bool    q5   = type == TYPE_Q5_K;
+    auto          kern = M == 1 ? (q5 ? k_gemv_q45_q6_norm<1, true> : k_gemv_q45_q6_norm<1, false>)
+                                : (q5 ? k_gemv_q45_q6_norm<2, true> : k_gemv_q45_q6_norm<2, false>);
+    hipLaunchKernelGGL(kern, dim3((unsigned) (na + nv)), dim3(64 * PG_WAVES), 0, (hipStream_t) stream, a, v, (int) na);
+    return check_launch("rms_norm_mul_mat_pair");
 }
 
 extern "C" int mmhip_swiglu_mul_mat_supported(int type, int64_t N, int64_t K, int64_t M) {

@@ -84,3 +84,33 @@ def test_depth_layer_with_and_without(pkg, S, B):
     finally:
         del os.environ["GGML_MI355X_DISABLE_GEMV_MULTI"]
     assert np.isfinite(joined).all() and np.array_equal(joined, separate)
+
+
+@pytest.mark.parametrize("wt,M,N,N2", [(13, 2, 5120, 1024), (12, 1, 5120, 1024), (13, 1, 300, 40), (12, 2, 17, 9001),
+                                       (13, 2, 30000, 5)])
+def test_pair_equals_separate(mm, pkg, wt, M, N, N2):
+    """A Q4_K / Q5_K and a Q6_K GEMV on the same normed rows in one launch
+    (mmhip_rms_norm_mul_mat_pair), bit for bit the two launches: one row to
+    several row iterations on either side, ragged row counts."""
+    L = mm.load()
+    K = 4096
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    W = mm.QuantWeight.from_gguf(wt, pkg.synth.gguf_blocks_np(wt, N, K, 61), N, K)
+    V = mm.QuantWeight.from_gguf(mm.Q6_K, pkg.synth.gguf_blocks_np(mm.Q6_K, N2, K, 62), N2, K)
+    x = torch.from_numpy(pkg.synth.normal_np((M, K), 63)).cuda() * 2
+    nw = torch.from_numpy(1 + 0.05 * pkg.synth.normal_np((1, K), 64)).cuda()
+    ref = []
+    for w in (W, V):
+        y = torch.empty((M, w.N), device="cuda")
+        assert L.mmhip_rms_norm_mul_mat(w.qtype, ptr(w.data), w.N, K, w.row_bytes, ptr(x), K, M, ptr(nw), 1e-6, None,
+                                        None, 0, ptr(y), w.N, st) == 0
+        ref.append(y)
+    y = torch.full((M, N + 4), float("nan"), device="cuda")
+    v = torch.full((M, N2 + 8), float("nan"), device="cuda")
+    assert L.mmhip_rms_norm_mul_mat_pair_supported(wt, N, mm.Q6_K, N2, K, M) == 1
+    assert L.mmhip_rms_norm_mul_mat_pair(wt, ptr(W.data), N, W.row_bytes, ptr(y), N + 4, mm.Q6_K, ptr(V.data), N2,
+                                         V.row_bytes, ptr(v), N2 + 8, K, ptr(x), K, M, ptr(nw), 1e-6, st) == 0
+    assert torch.equal(y[:, :N], ref[0]) and torch.equal(v[:, :N2], ref[1])
+    assert torch.isnan(y[:, N:]).all() and torch.isnan(v[:, N2:]).all()
+    for t2, k, m in [(mm.Q6_K, 2048, 2), (mm.Q6_K, 4096, 3), (wt, 4096, 2)]:
+        assert L.mmhip_rms_norm_mul_mat_pair_supported(wt, N, t2, N2, k, m) == 0
