@@ -579,30 +579,71 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_q(const uint8_t * __restrict__
 
 // Split-K reduction: y[m, n] = ((part_0 + part_1 + ...) + bias[n]) + res[m, n],
 // the parts summed in order, each ADD rounded as its op; 4 columns per thread.
-__global__ void k_splitk_reduce(const float * __restrict__ part, int nparts, int64_t M, int64_t N,
-                                const float * __restrict__ bias, const float * res, int64_t ldr, float * y,
-                                int64_t ldy) {
+// Bound by memory (every part read once): NP > 0 parts are loaded together,
+// one wait for all of a thread's loads instead of one a part, and VEC reads
+// and writes whole 16-byte groups (res, y and bias 16-byte aligned rows).
+// Four parts of 1380 x 2048 with both ADDs: 18.2 -> 11.2 us (6.0 TB/s).
+template <int NP, bool VEC>
+__global__ __launch_bounds__(256) void k_splitk_reduce(const float * __restrict__ part, int nparts, int64_t M, int64_t N,
+                                                       const float * __restrict__ bias, const float * res, int64_t ldr,
+                                                       float * y, int64_t ldy) {
 #pragma clang fp contract(off)
-    const int64_t n4 = N / 4;
-    for (int64_t t = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; t < M * n4; t += (int64_t) gridDim.x * blockDim.x) {
-        const int64_t m = t / n4, n = (t % n4) * 4;
-        float4_t      v = *(const float4_t *) (part + m * N + n);
-        for (int p = 1; p < nparts; p++) {
-            const float4_t w = *(const float4_t *) (part + ((int64_t) p * M + m) * N + n);
-            v[0]             = v[0] + w[0];
-            v[1]             = v[1] + w[1];
-            v[2]             = v[2] + w[2];
-            v[3]             = v[3] + w[3];
-        }
+    const int64_t n4 = N / 4, nt = M * n4;
+    for (int64_t t = blockIdx.x * (int64_t) blockDim.x + threadIdx.x; t < nt; t += (int64_t) gridDim.x * blockDim.x) {
+        const int64_t m = nt < (1ll << 32) ? (uint32_t) t / (uint32_t) n4 : t / n4;
+        const int64_t n = (t - m * n4) * 4;
+        float4_t      w[NP > 0 ? NP : 1], bv = { 0.0f, 0.0f, 0.0f, 0.0f }, rv = bv;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            if (bias) {
-                v[k] = v[k] + bias[n + k];
-            }
+        for (int p = 0; p < (NP > 0 ? NP : 1); p++) {
+            w[p] = *(const float4_t *) (part + ((int64_t) p * M + m) * N + n);
+        }
+        if constexpr (VEC) {
             if (res) {
-                v[k] = res[m * ldr + n + k] + v[k];
+                rv = *(const float4_t *) (res + m * ldr + n);
             }
-            y[m * ldy + n + k] = v[k];
+            if (bias) {
+                bv = *(const float4_t *) (bias + n);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                rv[k] = res ? res[m * ldr + n + k] : 0.0f;
+                bv[k] = bias ? bias[n + k] : 0.0f;
+            }
+        }
+        float4_t v = w[0];
+        auto     add = [&](const float4_t & o) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] = v[k] + o[k];
+            }
+        };
+        if constexpr (NP > 0) {
+#pragma unroll
+            for (int p = 1; p < NP; p++) {
+                add(w[p]);
+            }
+        } else {
+            for (int p = 1; p < nparts; p++) {
+                add(*(const float4_t *) (part + ((int64_t) p * M + m) * N + n));
+            }
+        }
+        if (bias) {
+            add(bv);
+        }
+        if (res) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                v[k] = rv[k] + v[k];
+            }
+        }
+        if constexpr (VEC) {
+            *(float4_t *) (y + m * ldy + n) = v;
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                y[m * ldy + n + k] = v[k];
+            }
         }
     }
 }
@@ -795,8 +836,19 @@ static int splitk_reduce(const GemmSplit & spl, int64_t M, int64_t N, const floa
                          int64_t ldr, float * y, int64_t ldy, hipStream_t stream) {
     const int64_t nt = M * (N / 4);
     const int64_t nb = (nt + 255) / 256;
-    hipLaunchKernelGGL(k_splitk_reduce, dim3((unsigned) (nb < 16384 ? nb : 16384)), dim3(256), 0, stream,
-                       (const float *) spl.part, spl.n, M, N, bias, res, ldr, y, ldy);
+    auto          al = [](const float * p, int64_t ld) { return ((uintptr_t) p) % 16 == 0 && ld % 4 == 0; };
+    const bool    vec = al(y, ldy) && (!res || al(res, ldr)) && (!bias || al(bias, 0));
+    auto          kern = vec ? k_splitk_reduce<0, true> : k_splitk_reduce<0, false>;
+    if (vec) {
+        switch (spl.n) {
+            case 2: kern = k_splitk_reduce<2, true>; break;
+            case 3: kern = k_splitk_reduce<3, true>; break;
+            case 4: kern = k_splitk_reduce<4, true>; break;
+            default: break;
+        }
+    }
+    hipLaunchKernelGGL(kern, dim3((unsigned) (nb < 16384 ? nb : 16384)), dim3(256), 0, stream, (const float *) spl.part,
+                       spl.n, M, N, bias, res, ldr, y, ldy);
     return check_launch("mul_mat gemm: split-K reduce");
 }
 
