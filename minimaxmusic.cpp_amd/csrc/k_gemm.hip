@@ -1,14 +1,17 @@
-// k_gemm.hip - MUL_MAT at token counts (M > 16): MFMA GEMM with the weight
-// tile dequantised into LDS.
+// k_gemm.hip - MUL_MAT at token counts (M > 16): the choice of kernel, the
+// conversions around it, and the kernels of many tokens.
 //
 //   y[m, n] = sum_k x[m, k] * deq(W)[n, k]
 //
 // The activations are first rounded to f16 into a packed copy (workspace):
 // every workgroup along N reads them, so they are converted once and moved at
-// half the bytes.  Workgroup tile: 256 tokens x 256 weight rows (8 waves,
-// each 128 x 64 with eight v_mfma_f32_32x32x16_f16 accumulators) when the
-// problem has at least 256 such tiles, else 64 tokens x 128 weight rows (4
-// waves, each 32 x 64); K step 64.  The weight tile is dequantised exactly as the GGUF
+// half the bytes.  Few tokens run k_gemm_sk, the middle counts k_gemm_p (each
+// in its own file, with the rule that takes a shape to it); here are the
+// kernels of full grids: 256 tokens x 256 weight rows, DMA'd from f16 rows
+// (four waves of 128 x 128) or with the weight tile dequantised through
+// registers (eight waves of 128 x 64), and 64 tokens x 128 rows (four waves
+// of 32 x 64) for f16 rows on small grids and for Q8_0 rows whose width is no
+// multiple of 256.  The weight tile is dequantised exactly as the GGUF
 // definitions (f32, no contraction) and then rounded to f16; both tiles are
 // k-contiguous rows in LDS, the operand order of the MFMA A (tokens) and B
 // (weight rows) inputs.  The output accumulator layout gives each lane one
@@ -253,7 +256,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_q(const uint8_t * __restrict__
     static_assert(MB >= 1 && XI >= 1, "tile shape");
     static_assert(!WH || BK == 32, "the f16-weight ring steps 32 columns");
     static_assert(!GLU || NB % 2 == 0, "GLU tiles pair value and gate blocks in each wave");
-    static_assert(!WIDE || (WH && NW == 4 && (BM == 256 || BM == 192)), "the wide tiles run on the DMA ring, four waves");
+    static_assert(!WIDE || (WH && NW == 4 && BM == 256), "the wide tiles run on the DMA ring, four waves");
     extern __shared__ __attribute__((aligned(16))) _Float16 g_lds[];
     _Float16 * sX = g_lds;            // 2 stages
     _Float16 * sW = g_lds + 2 * TIX;  // 2 buffers

@@ -11,6 +11,12 @@
 // dequantised between the MFMAs, once per tile.  Each of the step's four
 // 16-column products has its operands read during the product before, so the
 // step has one barrier, placed before its last product.
+//
+// What bounds it: the dequantisation's VALU work, the LDS operand reads and
+// the MFMAs, which overlap in part only (a wave's step waits on all three).
+// A layer's four projections at 333 tokens, Q6_K: 555 us on 64 x 128 tiles,
+// which dequantised every weight six times, -> 301 us; the DiT block's f16
+// copies at 1380 tokens: q / k / v 60 -> 57 us, ff_in 127 -> 125.
 #include "k_gemm_common.h"
 
 namespace mmhip {

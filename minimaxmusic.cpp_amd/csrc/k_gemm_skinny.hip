@@ -17,6 +17,10 @@
 // and the epilogue (bias, residual, or the SwiGLU of value / gate rows) runs
 // on the sums: no workspace and no second launch, and the same sums for every
 // form of the call.
+//
+// A layer's four projections (6144, 4096, 24576 rows of 4096, 4096 of 12288)
+// at 40 tokens, Q8_0, 220 MB of weights: 272 us on tiles -> 102 us, 2.2 TB/s
+// (the copies of the activations, 4 x 4.7 us, included).
 #include "k_gemm_common.h"
 
 namespace mmhip {
