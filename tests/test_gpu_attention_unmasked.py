@@ -3,11 +3,11 @@ where the DMA kernel's tiles and units end: key counts round the 32-key unit,
 the 64-key tile and the 4-tile ring, ragged query tiles, one workgroup and
 more, grouped KV heads, strided K / V.
 
-Tolerance: Q, P and the products' f16 operands are rounded to 2^-11 of
-themselves, so against fp64 the output moves by at most 2^-11 (P) plus
-2^-11 log2(e)-free score error |s|_max (Q) of the weighted |V|; with |s| <= 6
-and |V| <= 5 that is 2^-11 * 7 * 5 = 0.017 at worst; the rounding errors being
-independent, 2e-3 (the bound of the other attention tests) holds by far."""
+Tolerance: the f16 roundings of Q (a score error of at most 2^-11 |s|) and of
+P (2^-11 of each weight) move the output by at most 2^-11 (|s| + 1) of the
+weighted |V|: 0.017 with |s| <= 6 and |V| <= 5 if every rounding went the same
+way.  They are independent, so 2e-3, the bound of the other attention tests,
+holds by far."""
 import numpy as np
 import pytest
 import torch
@@ -53,8 +53,7 @@ def test_running_max_moves(mm, D):
     v = rng.standard_normal((1, 2, nkv, D)).astype(np.float16)
     q16 = q.astype(np.float16).astype(np.float32)
     s = 0.5
-    # the oracle on f16 queries: a score error of |q| 2^-11 would not be small here;
-    # s = 0.5 keeps the kernel's scaled query one rounding (log2 e) from it
+    # queries that f16 holds exactly: the kernel rounds only their scaled form
     out = run(mm, q16, k, v, s)
     ref = oracle(q16, k, v, s)
     # scaled-query rounding: 2^-11 of each of D products of a score of up to ~200, summed
